@@ -549,8 +549,9 @@ int build_device(td1c_ctx* c) {
     }
     HIP_TRY(c->b_L2g.upload(flat_or_one(b)));
     b.clear();
-    // gorbg and v2orbg (contiguous) -> gorb and v2orb (contiguous)
-    for (int w = 0; w < 2; ++w)
+    // gorbg and v2orbg (contiguous) -> gorb and v2orb (contiguous); without
+    // active orbitals v2 is zero: v2orb keeps the zeros written above
+    for (int w = 0; w < (S.nact > 0 ? 2 : 1); ++w)
       for (int f = nfc; f < nf; ++f) {
         int d = w * c->nd + (f - nfc);
         b.push_back({(long long)(d * ng), 0, (long long)(d * nb), S.mval[f] + S.mmax1, nr});
@@ -560,15 +561,18 @@ int build_device(td1c_ctx* c) {
   }
 
   // Gram products over the l-space basis: left = orb_0..orb_{nf-1}, h01 of
-  // frozen core; right = h01, gorb, v2orb, orb of the dynamical orbitals.
+  // frozen core; right = h01, gorb, v2orb (with active orbitals; zero
+  // otherwise) and orb (with frozen cores) of the dynamical orbitals.
   {
     std::vector<const void*> L, R;
     for (int f = 0; f < nf; ++f) L.push_back(c->orb + (size_t)f * nb);
     for (int f = 0; f < nfc; ++f) L.push_back(c->h01 + (size_t)f * nb);
     for (int f = nfc; f < nf; ++f) R.push_back(c->h01 + (size_t)f * nb);
     for (int d = 0; d < c->nd; ++d) R.push_back(c->gorb + (size_t)d * nb);
-    for (int d = 0; d < c->nd; ++d) R.push_back(c->v2orb + (size_t)d * nb);
-    for (int f = nfc; f < nf; ++f) R.push_back(c->orb + (size_t)f * nb);
+    const int nV = S.nact > 0 ? c->nd : 0;  // v2 columns
+    for (int d = 0; d < nV; ++d) R.push_back(c->v2orb + (size_t)d * nb);
+    if (nfc > 0)
+      for (int f = nfc; f < nf; ++f) R.push_back(c->orb + (size_t)f * nb);
     c->gl_nL = (int)L.size();
     c->gl_nR = (int)R.size();
     if (c->gl_nL * c->gl_nR > kMaxGram) return fail(-2, "too many orbitals for the Gram kernel");
@@ -582,8 +586,8 @@ int build_device(td1c_ctx* c) {
         int di = i - nfc;
         mH[j * nf + i] = 2 * (j * nR + di);
         mG[j * nf + i] = 2 * (j * nR + nd + di);
-        mV[j * nf + i] = 2 * (j * nR + 2 * nd + di);
-        if (j < nfc) mF[j * nf + i] = 2 * ((nf + j) * nR + 3 * nd + di);
+        if (nV > 0) mV[j * nf + i] = 2 * (j * nR + 2 * nd + di);
+        if (j < nfc) mF[j * nf + i] = 2 * ((nf + j) * nR + 2 * nd + nV + di);
       }
     HIP_TRY(c->mapH.upload(mH));
     HIP_TRY(c->mapG.upload(mG));
@@ -931,7 +935,7 @@ DtorbArgs dtorb_args(td1c_ctx* c, double dtime) {
   Setup& S = c->S;
   DtorbArgs d{};
   d.nbas = c->nbas; d.nr = S.nr; d.nfun = S.nfun; d.nfcore = S.nfcore;
-  d.mval = c->mval.p; d.h01 = c->h01; d.gorb = c->gorb; d.v2orb = c->v2orb; d.orb = c->orb; d.xmat = c->xmat.p;
+  d.mval = c->mval.p; d.h01 = c->h01; d.gorb = c->gorb; d.v2orb = S.nact > 0 ? c->v2orb : nullptr; d.orb = c->orb; d.xmat = c->xmat.p;
   d.tfac = S.icomp == 0 ? make_double2(-dtime, 0.0) : make_double2(0.0, -dtime);
   d.xlocal = c->x_local ? 1 : 0;
   d.ncore = S.ncore;

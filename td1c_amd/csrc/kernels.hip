@@ -1027,7 +1027,7 @@ __device__ __forceinline__ void mfprod_body(const A2* __restrict__ orbg, const A
   }
   for (int f = nfc; f < a.nfun; ++f) {
     gorbg[(size_t)(f - nfc) * ng + g] = ag[f];
-    v2orbg[(size_t)(f - nfc) * ng + g] = av[f];
+    if (na > 0) v2orbg[(size_t)(f - nfc) * ng + g] = av[f];  // zero without active orbitals: not formed
   }
 }
 
@@ -1136,7 +1136,7 @@ __device__ __forceinline__ void mfprod_t_body(const A2* __restrict__ orbg, const
 #pragma unroll
   for (int f = NFC; f < NF; ++f) {
     gorbg[(size_t)(f - NFC) * ng + g] = ag[f];
-    v2orbg[(size_t)(f - NFC) * ng + g] = av[f];
+    if (NA > 0) v2orbg[(size_t)(f - NFC) * ng + g] = av[f];
   }
 }
 
@@ -1439,13 +1439,9 @@ __device__ __forceinline__ void dtorb_body(const DtorbArgs& a, const Blk bk) {
   double2 k = make_double2(0.0, 0.0);
   if (f >= a.nfcore) {
     const size_t di = (size_t)(f - a.nfcore) * nb + q;
-    double2 h;
-    if (a.isplit == 1) {
-      h = cadd(a.v2orb[di], a.gorb[di]);
-    } else {
-      h = a.h01[idx];
-      h = cadd(a.v2orb[di], cadd(a.gorb[di], h));
-    }
+    double2 h = a.gorb[di];
+    if (a.isplit != 1) h = cadd(h, a.h01[idx]);
+    if (a.v2orb) h = cadd(a.v2orb[di], h);
     k = cmul(h, a.tfac);
     for (int j = 0; j < a.nfun; ++j) {
       if (a.mval[j] != a.mval[f]) continue;

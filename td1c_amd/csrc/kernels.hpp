@@ -155,7 +155,7 @@ struct GramArgs {
 struct DtorbArgs {
   int nbas, nr, nfun, nfcore;
   const int* mval;
-  const double2 *h01, *gorb, *v2orb, *orb, *xmat;
+  const double2 *h01, *gorb, *v2orb, *orb, *xmat;  // v2orb: null without active orbitals (v2 is zero)
   double2 tfac;
   // xlocal: each block builds its column of X from the l-space Gram products
   // (fc-dyn, core-core and active-active blocks; no core-active block, i.e.
