@@ -92,6 +92,8 @@ struct td1c_ctx {
   DevBuf<double2> tdiag, tzor;
   DevBuf<double> eK0, eK, eP;
   DevBuf<double> m_l2g, m_g2l, m_g2L, m_L2g;
+  DevBuf<double> k_l2g, k_g2l, k_g2L, k_L2g;  // packed for the matrix cores
+  LegendreMats t_l2g{}, t_g2l{}, t_g2L{}, t_L2g{};
   DevBuf<double> pG, pWl, pWr, pWlI, pWrI, pcrA, pcrG, pcrBinv, pSd, pSl, pSu, invr, rpl0, rpl1, fac2, fac1;
   DevBuf<int> mval, lval, pair_m, pj, pi, ptype, emap;
   // batches
@@ -106,7 +108,7 @@ struct td1c_ctx {
   bool mixed = false;
   DevBuf<float2> gsp_f, rhoL_f, vL_f, vg_f;
   float2 *orbg_f = nullptr, *gorbg_f = nullptr, *v2orbg_f = nullptr;
-  DevBuf<float> m_g2L_f, m_L2g_f;
+  DevBuf<float> m_g2L_f, m_L2g_f, k_g2L_f, k_L2g_f;
   DevBuf<double2> orbg0;     // frozen-core theta-grid orbitals at A = 0
   DevBuf<double2> rhoL, vL, vg;
   DevBuf<double2> p_xb, p_Q;  // Poisson bridge solutions [pair][L][nfe-1], multipole moments [pair][L]
@@ -164,10 +166,8 @@ struct td1c_ctx {
   // launch shape of the element one-body kernel (autotuned per problem):
   // elements per block (0: 3, 1: 6, 2: 12) and l values per block
   int ob_shape = 2, ob_lc = 2;
-  // launch shape of the register-blocked matrix-core transforms (0..5;
-  // TD1C_TVAR in the environment overrides it): 1 = 2 column tiles per
-  // wavefront, 4 contraction steps per load batch, measured best on the Ar
-  // workload among (4,4) (2,4) (4,8) (8,4) (8,2) (2,8)
+  // rows per block of the matrix-core transforms (0: 32, in a batch 16; else
+  // 16, in a batch 8); TD1C_TVAR in the environment overrides it
   int tvar = 1;
   std::string tune_log;  // what the autotuner measured (JSON)
   // device-driven propagation: one captured RK step, replayed per step
@@ -224,7 +224,7 @@ struct td1c_ctx {
   std::vector<std::pair<std::string, std::pair<double, int>>> timing_agg;
 
   ~td1c_ctx() {
-    DevBuf<double>* d[] = {&eK0, &eK, &eP, &xr, &band_k, &band_k0, &band_p, &alph, &cost, &mask, &m_l2g, &m_g2l, &m_g2L, &m_L2g,
+    DevBuf<double>* d[] = {&eK0, &eK, &eP, &xr, &band_k, &band_k0, &band_p, &alph, &cost, &mask, &m_l2g, &m_g2l, &m_g2L, &m_L2g, &k_l2g, &k_g2l, &k_g2L, &k_L2g,
                            &pG, &pWl, &pWr, &pWlI, &pWrI, &pcrA, &pcrG, &pcrBinv, &pSd, &pSl, &pSu, &invr, &rpl0, &rpl1, &fac2, &fac1, &ene, &lf_dev,
                        &cn_part, &lf_cn};
     for (auto* b : d) b->release();
@@ -246,7 +246,7 @@ struct td1c_ctx {
     b_g2l_gfc.release();
     dip3_tmp.release();
     for (auto* b : ff) b->release();
-    DevBuf<float>* fm[] = {&m_g2L_f, &m_L2g_f};
+    DevBuf<float>* fm[] = {&m_g2L_f, &m_L2g_f, &k_g2L_f, &k_L2g_f};
     for (auto* b : fm) b->release();
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (cn_flag_host) (void)hipHostFree(cn_flag_host);
@@ -387,6 +387,26 @@ std::vector<double> padded_cols(const std::vector<double>& m, int K, int C) {
   return out;
 }
 
+// [nm][K][C] -> the packed operands of LegendreMats; matrix index = m + mmax
+std::vector<double> packed_legendre(const std::vector<double>& m, int K, int C, int mmax, bool analysis) {
+  const int KS = legendre_steps(K), MT = legendre_tiles(C), nm = 2 * mmax + 1;
+  const int KH = (K + 1) / 2, CH = (C + 1) / 2;
+  std::vector<double> out((size_t)nm * 2 * KS * MT * 64, 0.0);
+  size_t q = 0;
+  for (int i = 0; i < nm; ++i)
+    for (int cls = 0; cls < 2; ++cls) {
+      const int odd = (cls + std::abs(i - mmax)) & 1;
+      for (int ks = 0; ks < KS; ++ks)
+        for (int mt = 0; mt < MT; ++mt)
+          for (int lane = 0; lane < 64; ++lane, ++q) {
+            const int kk = 4 * ks + lane / 16, cc = 16 * mt + lane % 16;
+            const int k = analysis ? kk : 2 * kk + odd, c = analysis ? 2 * cc + odd : cc;
+            if (analysis ? (kk < KH && c < C) : (k < K && cc < CH)) out[q] = m[((size_t)i * K + k) * C + c];
+          }
+    }
+  return out;
+}
+
 OneBodyElArgs onebody_el_args(td1c_ctx* c, const double* d_lf) {
   const Setup& S = c->S;
   OneBodyElArgs oe{};
@@ -433,6 +453,12 @@ int build_device(td1c_ctx* c) {
   HIP_TRY(c->m_g2l.upload(padded_cols(S.mat_g2l, S.nlat, S.L1)));
   HIP_TRY(c->m_g2L.upload(padded_cols(S.mat_g2L, S.nlat, S.L2)));
   HIP_TRY(c->m_L2g.upload(padded_cols(S.mat_L2g, S.L2, S.nlat)));
+  const std::vector<double> pk_g2L = packed_legendre(S.mat_g2L, S.nlat, S.L2, S.mmax2, true);
+  const std::vector<double> pk_L2g = packed_legendre(S.mat_L2g, S.L2, S.nlat, S.mmax2, false);
+  HIP_TRY(c->k_l2g.upload(packed_legendre(S.mat_l2g, S.L1, S.nlat, S.mmax1, false)));
+  HIP_TRY(c->k_g2l.upload(packed_legendre(S.mat_g2l, S.nlat, S.L1, S.mmax1, true)));
+  HIP_TRY(c->k_g2L.upload(pk_g2L));
+  HIP_TRY(c->k_L2g.upload(pk_L2g));
   {
     // element inverses G_e stored transposed on the device, [L][e][k][i]:
     // lanes owning consecutive rows i read consecutive addresses
@@ -512,7 +538,13 @@ int build_device(td1c_ctx* c) {
     std::vector<double> g2L = padded_cols(S.mat_g2L, S.nlat, S.L2), L2g = padded_cols(S.mat_L2g, S.L2, S.nlat);
     HIP_TRY(c->m_g2L_f.upload(std::vector<float>(g2L.begin(), g2L.end())));
     HIP_TRY(c->m_L2g_f.upload(std::vector<float>(L2g.begin(), L2g.end())));
+    HIP_TRY(c->k_g2L_f.upload(std::vector<float>(pk_g2L.begin(), pk_g2L.end())));
+    HIP_TRY(c->k_L2g_f.upload(std::vector<float>(pk_L2g.begin(), pk_L2g.end())));
   }
+  c->t_l2g = {0, S.L1, S.nlat, c->m_l2g.p, c->k_l2g.p, nullptr, nullptr};
+  c->t_g2l = {1, S.nlat, S.L1, c->m_g2l.p, c->k_g2l.p, nullptr, nullptr};
+  c->t_g2L = {1, S.nlat, S.L2, c->m_g2L.p, c->k_g2L.p, c->m_g2L_f.p, c->k_g2L_f.p};
+  c->t_L2g = {0, S.L2, S.nlat, c->m_L2g.p, c->k_L2g.p, c->m_L2g_f.p, c->k_L2g_f.p};
   HIP_TRY(c->orbg0.alloc(std::max<size_t>(1, ng * nfc)));
   HIP_TRY(hipMemset(c->orbg0.p, 0, c->orbg0.n * sizeof(double2)));
   const size_t np = np0;
@@ -523,12 +555,12 @@ int build_device(td1c_ctx* c) {
   {
     std::vector<TransformBatch> b;
     for (int f = nfc; f < nf; ++f)
-      b.push_back({(long long)(f * nb), 0, (long long)(f * ng), S.mval[f] + S.mmax1, nr});
+      b.push_back({(long long)(f * nb), 0, (long long)(f * ng), S.mval[f] + S.mmax1, nr, std::abs(S.mval[f]) & 1});
     c->n_l2g_dyn = (int)b.size();
     HIP_TRY(c->b_l2g_dyn.upload(b));
     b.clear();
     for (int f = 0; f < nfc; ++f)
-      b.push_back({(long long)(f * ng), 0, (long long)(f * nb), S.mval[f] + S.mmax1, S.nradfc});
+      b.push_back({(long long)(f * ng), 0, (long long)(f * nb), S.mval[f] + S.mmax1, S.nradfc, std::abs(S.mval[f]) & 1});
     c->n_g2l_fc = (int)b.size();
     HIP_TRY(c->b_g2l_fc.upload(flat_or_one(b)));
     b.clear();
@@ -537,7 +569,7 @@ int build_device(td1c_ctx* c) {
       auto& p = S.pairs[q];
       int mji = S.mval[p.i] - S.mval[p.j];
       b.push_back({(long long)(p.j * ng), (long long)(p.i * ng), (long long)((size_t)q * L2 * nr), mji + S.mmax2,
-                   p.type == 1 ? S.nradfc : nr});
+                   p.type == 1 ? S.nradfc : nr, std::abs(mji) & 1});
     }
     HIP_TRY(c->b_rho.upload(flat_or_one(b)));
     b.clear();
@@ -545,7 +577,7 @@ int build_device(td1c_ctx* c) {
       auto& p = S.pairs[q];
       int mji = S.mval[p.i] - S.mval[p.j];
       b.push_back({(long long)((size_t)q * L2 * nr), 0, (long long)((size_t)q * nl * nr), mji + S.mmax2,
-                   p.type == 1 ? S.nradfc : nr});
+                   p.type == 1 ? S.nradfc : nr, std::abs(mji) & 1});
     }
     HIP_TRY(c->b_L2g.upload(flat_or_one(b)));
     b.clear();
@@ -554,7 +586,7 @@ int build_device(td1c_ctx* c) {
     for (int w = 0; w < (S.nact > 0 ? 2 : 1); ++w)
       for (int f = nfc; f < nf; ++f) {
         int d = w * c->nd + (f - nfc);
-        b.push_back({(long long)(d * ng), 0, (long long)(d * nb), S.mval[f] + S.mmax1, nr});
+        b.push_back({(long long)(d * ng), 0, (long long)(d * nb), S.mval[f] + S.mmax1, nr, std::abs(S.mval[f]) & 1});
       }
     c->n_g2l_mf = (int)b.size();
     HIP_TRY(c->b_g2l_mf.upload(b));
@@ -764,11 +796,9 @@ void enqueue_orbin_theta(td1c_ctx* c, const double* d_lf, const double2* wfn, hi
   {
     TIMED("l2theta");
     if (c->mixed)
-      launch_transform_t<double2, float2>(0, wfn, c->orbg_f, c->m_l2g.p, nullptr, c->b_l2g_dyn.p, c->n_l2g_dyn, nr, L1,
-                                          nl, pad_cols(nl), c->orb, s, c->tpath, fc_vel ? &fj : nullptr, c->tvar);
+      launch_transform_t<double2, float2>(0, wfn, c->orbg_f, c->t_l2g, c->b_l2g_dyn.p, c->n_l2g_dyn, nr, c->orb, s, c->tpath, fc_vel ? &fj : nullptr, c->tvar);
     else
-      launch_transform_t<double2, double2>(0, wfn, c->orbg, c->m_l2g.p, nullptr, c->b_l2g_dyn.p, c->n_l2g_dyn, nr, L1,
-                                           nl, pad_cols(nl), c->orb, s, c->tpath, fc_vel ? &fj : nullptr, c->tvar);
+      launch_transform_t<double2, double2>(0, wfn, c->orbg, c->t_l2g, c->b_l2g_dyn.p, c->n_l2g_dyn, nr, c->orb, s, c->tpath, fc_vel ? &fj : nullptr, c->tvar);
   }
 }
 
@@ -779,11 +809,9 @@ void enqueue_orbin_fc_l(td1c_ctx* c, hipStream_t s) {
   if (nfc > 0 && S.igauge == 1) {
     TIMED_ON(s, "theta2l_fc");
     if (c->mixed)
-      launch_transform_t<float2, double2>(0, c->orbg_f, c->orb, c->m_g2l.p, nullptr, c->b_g2l_fc.p, c->n_g2l_fc, nr, nl,
-                                          L1, pad_cols(L1), nullptr, s, c->tpath, nullptr, c->tvar);
+      launch_transform_t<float2, double2>(0, c->orbg_f, c->orb, c->t_g2l, c->b_g2l_fc.p, c->n_g2l_fc, nr, nullptr, s, c->tpath, nullptr, c->tvar);
     else
-      launch_transform(0, c->orbg, c->orb, c->m_g2l.p, c->b_g2l_fc.p, c->n_g2l_fc, nr, nl, L1, pad_cols(L1), nullptr, s,
-                       c->tpath, nullptr, c->tvar);
+      launch_transform_t<double2, double2>(0, c->orbg, c->orb, c->t_g2l, c->b_g2l_fc.p, c->n_g2l_fc, nr, nullptr, s, c->tpath, nullptr, c->tvar);
   }
 }
 
@@ -844,11 +872,10 @@ int enqueue_htotx(td1c_ctx* c, double dtime, const double* d_lf, const double2* 
   if (S.nel[2] >= 2 && c->npair > 0) {
     if (c->mixed) {
       TIMED("pair_theta2L");
-      launch_transform_t<float2, float2>(1, c->orbg_f, c->rhoL_f.p, c->m_g2L.p, c->m_g2L_f.p, c->b_rho.p, c->npair, nr,
-                                         nl, L2, pad_cols(L2), nullptr, s, c->tpath, nullptr, c->tvar);
+      launch_transform_t<float2, float2>(1, c->orbg_f, c->rhoL_f.p, c->t_g2L, c->b_rho.p, c->npair, nr, nullptr, s, c->tpath, nullptr, c->tvar);
     } else {
       TIMED("pair_theta2L");
-      launch_transform(1, c->orbg, c->rhoL.p, c->m_g2L.p, c->b_rho.p, c->npair, nr, nl, L2, pad_cols(L2), nullptr, s, c->tpath, nullptr, c->tvar);
+      launch_transform_t<double2, double2>(1, c->orbg, c->rhoL.p, c->t_g2L, c->b_rho.p, c->npair, nr, nullptr, s, c->tpath, nullptr, c->tvar);
     }
     PoissonArgs pa{};
     pa.nr = nr; pa.n = S.n; pa.nfe = S.nfe; pa.ni = S.ni; pa.L2 = L2; pa.npair = c->npair;
@@ -865,15 +892,14 @@ int enqueue_htotx(td1c_ctx* c, double dtime, const double* d_lf, const double2* 
       pair_gram_done = true;
       {
         TIMED("pair_L2theta");
-        launch_transform_t<float2, float2>(0, c->vL_f.p, c->vg_f.p, c->m_L2g.p, c->m_L2g_f.p, c->b_L2g.p, c->npair, nr,
-                                           L2, nl, pad_cols(nl), nullptr, s, c->tpath, nullptr, c->tvar);
+        launch_transform_t<float2, float2>(0, c->vL_f.p, c->vg_f.p, c->t_L2g, c->b_L2g.p, c->npair, nr, nullptr, s, c->tpath, nullptr, c->tvar);
       }
     } else {
       { TIMED("poisson_bridge"); launch_poisson(c->rhoL.p, c->p_xb.p, c->vL.p, pa, s, 1); }
       { TIMED("poisson_interior"); launch_poisson(c->rhoL.p, c->p_xb.p, c->vL.p, pa, s, 2); }
       HIP_TRY(enqueue_pair_gram(c, s, s1));
       pair_gram_done = true;
-      { TIMED("pair_L2theta"); launch_transform(0, c->vL.p, c->vg.p, c->m_L2g.p, c->b_L2g.p, c->npair, nr, L2, nl, pad_cols(nl), nullptr, s, c->tpath, nullptr, c->tvar); }
+      { TIMED("pair_L2theta"); launch_transform_t<double2, double2>(0, c->vL.p, c->vg.p, c->t_L2g, c->b_L2g.p, c->npair, nr, nullptr, s, c->tpath, nullptr, c->tvar); }
     }
     MfArgs ma{};
     ma.nr = nr; ma.nlat = nl; ma.nfun = nf; ma.nfcore = nfc; ma.nfcore2 = S.nfcore2; ma.ncore = S.ncore; ma.nact = S.nact;
@@ -886,12 +912,11 @@ int enqueue_htotx(td1c_ctx* c, double dtime, const double* d_lf, const double2* 
       { TIMED("mfprod"); launch_mfprod(c->orbg_f, c->vg_f.p, c->gorbg_f, c->v2orbg_f, ma, s); }
       {
         TIMED("theta2l_mf");
-        launch_transform_t<float2, double2>(0, c->gorbg_f, c->gorb, c->m_g2l.p, nullptr, c->b_g2l_mf.p, c->n_g2l_mf, nr,
-                                            nl, L1, pad_cols(L1), nullptr, s, c->tpath, nullptr, c->tvar);
+        launch_transform_t<float2, double2>(0, c->gorbg_f, c->gorb, c->t_g2l, c->b_g2l_mf.p, c->n_g2l_mf, nr, nullptr, s, c->tpath, nullptr, c->tvar);
       }
     } else {
       { TIMED("mfprod"); launch_mfprod(c->orbg, c->vg.p, c->gorbg, c->v2orbg, ma, s); }
-      { TIMED("theta2l_mf"); launch_transform(0, c->gorbg, c->gorb, c->m_g2l.p, c->b_g2l_mf.p, c->n_g2l_mf, nr, nl, L1, pad_cols(L1), nullptr, s, c->tpath, nullptr, c->tvar); }
+      { TIMED("theta2l_mf"); launch_transform_t<double2, double2>(0, c->gorbg, c->gorb, c->t_g2l, c->b_g2l_mf.p, c->n_g2l_mf, nr, nullptr, s, c->tpath, nullptr, c->tvar); }
     }
   } else {
     launch_zero(c->gorb, 2 * nb * c->nd, s);
@@ -1328,10 +1353,10 @@ int td1c_set_wfn0(td1c_ctx* c, const double* wfn, const double* cic, const doubl
   {
     std::vector<TransformBatch> b;
     for (int f = 0; f < nfc; ++f)
-      b.push_back({(long long)(f * nb), 0, (long long)(f * (size_t)c->ngrid), S.mval[f] + S.mmax1, S.nradfc});
+      b.push_back({(long long)(f * nb), 0, (long long)(f * (size_t)c->ngrid), S.mval[f] + S.mmax1, S.nradfc, std::abs(S.mval[f]) & 1});
     DevBuf<TransformBatch> tb;
     HIP_TRY(tb.upload(b));
-    launch_transform(0, c->orb, c->orbg0.p, c->m_l2g.p, tb.p, nfc, nr, L1, S.nlat, pad_cols(S.nlat), nullptr, nullptr);
+    launch_transform_t<double2, double2>(0, c->orb, c->orbg0.p, c->t_l2g, tb.p, nfc, nr, nullptr, nullptr);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipDeviceSynchronize());
     tb.release();
@@ -1352,11 +1377,11 @@ int td1c_set_wfn0(td1c_ctx* c, const double* wfn, const double* cic, const doubl
     DevBuf<TransformBatch> tb;
     std::vector<TransformBatch> b;
     for (int f = 0; f < nfc; ++f)
-      b.push_back({(long long)(f * (size_t)c->ngrid), 0, (long long)(f * nb), S.mval[f] + S.mmax1, S.nradfc});
+      b.push_back({(long long)(f * (size_t)c->ngrid), 0, (long long)(f * nb), S.mval[f] + S.mmax1, S.nradfc, std::abs(S.mval[f]) & 1});
     HIP_TRY(tb.upload(b));
     DevBuf<double2> tmp;
     HIP_TRY(tmp.alloc(nb * nfc));
-    launch_transform(0, c->orbg0.p, tmp.p, c->m_g2l.p, tb.p, nfc, nr, S.nlat, L1, pad_cols(L1), nullptr, nullptr);
+    launch_transform_t<double2, double2>(0, c->orbg0.p, tmp.p, c->t_g2l, tb.p, nfc, nr, nullptr, nullptr);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipDeviceSynchronize());
     HIP_TRY(hipMemcpy(orbfc.data(), tmp.p, nb * nfc * sizeof(double2), hipMemcpyDeviceToHost));
@@ -1407,7 +1432,7 @@ int td1c_set_wfn0(td1c_ctx* c, const double* wfn, const double* cic, const doubl
       else HIP_TRY(c->gfc_g.alloc((size_t)2 * nfc * ng));
       std::vector<TransformBatch> b;
       for (int k = 0; k < 2 * nfc; ++k)
-        b.push_back({(long long)(k * ng), 0, (long long)(k * nb), S.mval[k % nfc] + S.mmax1, S.nradfc});
+        b.push_back({(long long)(k * ng), 0, (long long)(k * nb), S.mval[k % nfc] + S.mmax1, S.nradfc, std::abs(S.mval[k % nfc]) & 1});
       HIP_TRY(c->b_g2l_gfc.upload(b));
       DipoleFcArgs probe{};
       probe.nfun = S.nfun; probe.nfcore = nfc; probe.nradfc = S.nradfc; probe.L1 = S.L1;
@@ -1584,12 +1609,10 @@ int td1c_dipole_all(td1c_ctx* c, const double* lfield, const double* d_wfn, cons
   ga.vfc = c->vfc_tab.p;
   if (c->mixed) {
     launch_gfock_fc<float2>(c->orbg_f, c->vg_f.p, c->gfc_gf.p, ga, s);
-    launch_transform_t<float2, double2>(0, c->gfc_gf.p, c->gfc_l.p, c->m_g2l.p, nullptr, c->b_g2l_gfc.p, 2 * nfc, nr,
-                                        nl, L1, pad_cols(L1), nullptr, s, c->tpath, nullptr, c->tvar);
+    launch_transform_t<float2, double2>(0, c->gfc_gf.p, c->gfc_l.p, c->t_g2l, c->b_g2l_gfc.p, 2 * nfc, nr, nullptr, s, c->tpath, nullptr, c->tvar);
   } else {
     launch_gfock_fc<double2>(c->orbg, c->vg.p, c->gfc_g.p, ga, s);
-    launch_transform(0, c->gfc_g.p, c->gfc_l.p, c->m_g2l.p, c->b_g2l_gfc.p, 2 * nfc, nr, nl, L1, pad_cols(L1),
-                     nullptr, s, c->tpath, nullptr, c->tvar);
+    launch_transform_t<double2, double2>(0, c->gfc_g.p, c->gfc_l.p, c->t_g2l, c->b_g2l_gfc.p, 2 * nfc, nr, nullptr, s, c->tpath, nullptr, c->tvar);
   }
   DipoleArgs da{};
   da.nr = nr; da.L1 = L1; da.nfun = S.nfun; da.nfcore = nfc; da.ncore = S.ncore; da.nact = S.nact;
@@ -3398,6 +3421,8 @@ int batch_record(td1c_batch* b, const std::vector<Pulse>& pulses, int rk_order, 
                  int apply_mask) {
   const int nmem = (int)b->mem.size();
   std::vector<std::vector<LaunchRec>> recs(nmem);
+  int kmax = 0;  // the longest contraction decides the members' common transform shape (LDS)
+  for (td1c_ctx* c : b->mem) kmax = std::max({kmax, c->S.L2, c->S.nlat});
   for (int m = 0; m < nmem; ++m) {
     td1c_ctx* c = b->mem[m];
     int ns;
@@ -3409,7 +3434,7 @@ int batch_record(td1c_batch* b, const std::vector<Pulse>& pulses, int rk_order, 
     c->tpath = 2;  // the matrix-core transforms (their batched form)
     c->ob_shape = b->ob_shape;
     c->ob_lc = b->ob_lc;
-    c->tvar = b->tvar;
+    c->tvar = kmax > 200 ? 1 : b->tvar;
     c->capturing = true;  // no per-kernel timing events
     active_recorder() = &R;
     launch_field_stages(pulses[m], c->clock.p, sn, c->lf_dev.p, c->side[1]);

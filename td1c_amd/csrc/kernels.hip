@@ -132,15 +132,11 @@ __global__ void k_fc_phase(const FcPhaseJob j) {
 }
 
 // ---------------------------------------------------------------------------
-// The same transform on the matrix cores.  Per batch entry it is the real
-// GEMM Out^T = M^T X, with X[k][r] the complex input: its real and imaginary
-// parts are two MFMA B operands sharing the A operand (the real matrix).
-// Block: one tile of 16 radial rows and up to 4 column tiles of 16, one
-// wavefront per column tile, each running the whole contraction in steps of
-// 4 (MODE 1: over the pair products staged in LDS).  Lane layouts of the 16x16x4 MFMAs on
-// gfx950: A[i][k] at lane i + 16k, B[k][j] at lane j + 16k; register v of
-// the result in lane l holds column l % 16 and row 4 (l / 16) + v (f32) or
-// l / 16 + 4 v (f64).
+// The same transform on the matrix cores: the real GEMM Out^T = M^T X with
+// X[k][r] the complex input.  Lane layouts of the 16x16x4 MFMAs on gfx950:
+// A[i][k] at lane i + 16k, B[k][j] at lane j + 16k; register v of the result
+// in lane l holds column l % 16 and row 4 (l / 16) + v (f32) or l / 16 + 4 v
+// (f64).
 // ---------------------------------------------------------------------------
 template <class AR> struct Mfma16;
 template <> struct Mfma16<float> {
@@ -158,219 +154,198 @@ template <> struct Mfma16<double> {
   static __device__ __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
 };
 
-template <int MODE, class TI, class TO>
-__device__ __forceinline__ void transform_mfma_body(const TI* __restrict__ in, TO* __restrict__ out, const double* __restrict__ mats, const float* __restrict__ matsf, const TransformBatch* __restrict__ batch, int nr, int K, int C, int Cp, double2* __restrict__ copy, int nx, int ny, int ntile, const FcPhaseJob& fc, const Blk bk) {
+// Block: R = 8 NT radial rows of one batch entry, four wavefronts.  The
+// Legendre functions are even or odd about theta = pi/2 (P_l^m by l + m) and
+// the Gauss points are symmetric, so the contraction runs over half of the
+// theta points: theta -> l folds the input into S = x(k) + x(K-1-k) and
+// D = x(k) - x(K-1-k) for the even and odd l (the middle point of an odd K
+// enters both as it is), l -> theta forms E and O over the even and odd l and
+// writes E + O and E - O to the two mirror points.  That halves the matrix
+// work of the plain product.  The folded input of the block is staged in LDS
+// once ([class][k][row, re/im interleaved]) and serves every column tile;
+// the 16 columns of an MFMA tile are 8 radial rows times (re, im), so loads
+// and stores are whole segments of a radial row.  The matrices are packed
+// in operand order (LegendreMats), one coalesced load per step.  PAIR: the
+// input is the pair density conj(psi_j) psi_i of two theta-grid orbitals.
+// Bound: HBM, 439 MB per launch of 45 pairs x 127 x 2399 in FP64 (90 us at
+// the copy rate of 4.9 TB/s; the halved product takes 45 us of the FP64
+// matrix cores).  Measured in the step, us per launch against the plain
+// product (A operands re-read per row tile, no mirror symmetry): l -> theta
+// 139 against 190 (complex64 80 against 123), pair products theta -> l 126
+// against 181 (71 against 124); 9 orbitals l -> theta 21 against 30.  16 and
+// 32 rows per block are within 3 % of each other.
+template <class T> struct CScalar;
+template <> struct CScalar<double2> { using S = double; };
+template <> struct CScalar<float2> { using S = float; };
+
+template <bool AN, bool PAIR, int NT, class TI, class TO>
+__device__ __forceinline__ void legendre_body(const LegendreJob& J, const Blk bk) {
   using A2 = typename std::conditional<std::is_same<TI, float2>::value && std::is_same<TO, float2>::value, float2,
                                        double2>::type;
   using AR = typename CReal<A2>::T;
   using MF = Mfma16<AR>;
   using V4 = typename MF::V4;
-  constexpr int KC = 64;  // contraction values staged in LDS per pass
+  using SO = typename CScalar<TO>::S;
+  constexpr int R = 8 * NT, NC = 16 * NT, KPP = 256 / R;
+  extern __shared__ __align__(16) unsigned char leg_lds[];
   // blocks past the ntile transform tiles run the frozen-core phase job
-  if ((int)bk.x >= ntile) {
-    const int q = (int)bk.x - ntile, rb = (fc.nr + blockDim.x - 1) / blockDim.x;
-    fc_phase_point<TO>(fc, (q % rb) * blockDim.x + threadIdx.x, q / rb);
+  if ((int)bk.x >= J.ntile) {
+    const int q = (int)bk.x - J.ntile, rb = (J.fc.nr + 255) / 256;
+    fc_phase_point<TO>(J.fc, (q % rb) * 256 + threadIdx.x, q / rb);
     return;
   }
-  __shared__ A2 sX[MODE == 1 ? KC * 16 : 1];
-  const int t = xcd_remap(bk.x, ntile);
-  const int by = t % ny, bx = (t / ny) % nx, bz = t / (ny * nx);
-  const TransformBatch bt = batch[bz];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c0 = (by * (int)(blockDim.x >> 6) + wave) * 16;  // first column of this wavefront's tile
-  const bool active = c0 < C;  // wave-uniform
-  const int r0 = bx * 16;
-  const int kq = lane >> 4;
-  const int ca = c0 + (lane & 15);  // matrix column this lane feeds to A
-  const bool ca_ok = ca < Cp;       // columns C..Cp-1 of the padded matrix are zero
-  const AR* __restrict__ M;
-  if constexpr (std::is_same<AR, float>::value) M = matsf + (size_t)bt.mat * K * Cp;
-  else M = mats + (size_t)bt.mat * K * Cp;
-  V4 dre = {0, 0, 0, 0}, dim = {0, 0, 0, 0};
-  if constexpr (MODE == 1) {
-    // the pair products, formed once per block into LDS for all its
-    // column-tile wavefronts
-    for (int k0 = 0; k0 < K; k0 += KC) {
-      // stage: element q of the tile is (k = k0 + q / 16, row r0 + q % 16),
-      // four elements per thread per round with the loads issued together
-      for (int q0 = 0; q0 < KC * 16; q0 += 4 * (int)blockDim.x) {
-        TI x0[4], x1[4];
-        bool ok[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int q = q0 + u * (int)blockDim.x + (int)threadIdx.x;
-          const int k = k0 + (q >> 4), r = r0 + (q & 15);
-          ok[u] = q < KC * 16 && k < K && r < bt.rows;
-          const size_t g = (size_t)k * nr + r;
-          x0[u] = ok[u] ? in[(size_t)bt.in0 + g] : TI{};
-          x1[u] = ok[u] ? in[(size_t)bt.in1 + g] : TI{};
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int q = q0 + u * (int)blockDim.x + (int)threadIdx.x;
-          if (q < KC * 16) sX[q] = ok[u] ? cmulc(cto<A2>(x0[u]), cto<A2>(x1[u])) : cz<A2>();
-        }
-      }
-      __syncthreads();
-      if (active) {
-        const int nks = (min(KC, K - k0) + 3) >> 2;
-#pragma unroll 4
-        for (int st = 0; st < nks; ++st) {
-          const int kl = 4 * st + kq;
-          const int k = k0 + kl;
-          const AR a = (k < K && ca_ok) ? M[(size_t)k * Cp + ca] : AR(0);
-          const A2 x = sX[kl * 16 + (lane & 15)];
-          dre = MF::run(a, x.x, dre);
-          dim = MF::run(a, x.y, dim);
-        }
-      }
-      __syncthreads();
-    }
-  } else if (active) {
-    // plain input: each wavefront reads its B operand directly (the other
-    // column tiles of the block hit the same lines in L1)
-    constexpr int U = 4;  // contraction steps per load batch
-    const int r = r0 + (lane & 15);
-    const bool row_ok = r < bt.rows;
-    const TI* __restrict__ x0 = in + (size_t)bt.in0 + r;
-    const int nks = (K + 3) >> 2;
-    for (int s0 = 0; s0 < nks; s0 += U) {
-      AR a[U];
-      A2 x[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = 4 * (s0 + u) + kq;
-        const bool kok = k < K;
-        a[u] = (kok && ca_ok) ? M[(size_t)k * Cp + ca] : AR(0);
-        x[u] = cz<A2>();
-        if (kok && row_ok) {
-          const TI xv = x0[(size_t)k * nr];
-          x[u] = cto<A2>(xv);
-          if constexpr (std::is_same<TI, double2>::value)
-            if (copy != nullptr && c0 == 0) copy[(size_t)bt.in0 + (size_t)k * nr + r] = xv;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        dre = MF::run(a[u], x[u].x, dre);
-        dim = MF::run(a[u], x[u].y, dim);
-      }
-    }
-  }
-  const int r = r0 + (lane & 15);
-  if (active && r < bt.rows) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int c = c0 + MF::row(lane, v);
-      A2 o;
-      o.x = dre[v];
-      o.y = dim[v];
-      if (c < C) out[(size_t)bt.out + (size_t)c * nr + r] = cto<TO>(o);
-    }
-  }
-}
-
-template <int MODE, class TI, class TO>
-__global__ void __launch_bounds__(256) k_transform_mfma(const TI* __restrict__ in, TO* __restrict__ out,
-                                                        const double* __restrict__ mats,
-                                                        const float* __restrict__ matsf,
-                                                        const TransformBatch* __restrict__ batch, int nr, int K, int C,
-                                                        int Cp, double2* __restrict__ copy, int nx, int ny, int ntile,
-                                                        const FcPhaseJob fc) {
-  transform_mfma_body<MODE, TI, TO>(in, out, mats, matsf, batch, nr, K, C, Cp, copy, nx, ny, ntile, fc, hw_blk());
-}
-
-// The matrix-core transform with register blocking over columns: a
-// wavefront computes 16 radial rows x 16 CT columns, so that each input
-// value it loads (the MFMA B operand) feeds 2 CT MFMAs.  Block: four
-// wavefronts on consecutive row tiles sharing the same columns (their A
-// operands hit the same L1 lines).  Each output element is accumulated in
-// the same order as in k_transform_mfma, so both kernels give the same bits.
-template <int CT, int U, class TI, class TO>
-__device__ __forceinline__ void transform_mfma_w_body(const TI* __restrict__ in, TO* __restrict__ out, const double* __restrict__ mats, const float* __restrict__ matsf, const TransformBatch* __restrict__ batch, int nr, int K, int C, int Cp, double2* __restrict__ copy, int nx, int ny, int ntile, const FcPhaseJob& fc, const Blk bk) {
-  using A2 = typename std::conditional<std::is_same<TI, float2>::value && std::is_same<TO, float2>::value, float2,
-                                       double2>::type;
-  using AR = typename CReal<A2>::T;
-  using MF = Mfma16<AR>;
-  using V4 = typename MF::V4;
-  if ((int)bk.x >= ntile) {
-    const int q = (int)bk.x - ntile, rb = (fc.nr + blockDim.x - 1) / blockDim.x;
-    fc_phase_point<TO>(fc, (q % rb) * blockDim.x + threadIdx.x, q / rb);
-    return;
-  }
-  const int t = xcd_remap(bk.x, ntile);
-  const int by = t % ny, bx = (t / ny) % nx, bz = t / (ny * nx);
-  const TransformBatch bt = batch[bz];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c0 = by * 16 * CT;                   // first column of this wavefront's tiles
-  const int nct = min(CT, (C - c0 + 15) >> 4);   // its column tiles (wave-uniform)
-  const int r0 = (bx * 4 + wave) * 16;
-  const int kq = lane >> 4;
-  const int r = r0 + (lane & 15);
+  AR* sB = reinterpret_cast<AR*>(leg_lds);
+  const TI* __restrict__ in = static_cast<const TI*>(J.in);
+  const int t = xcd_remap(bk.x, J.ntile);
+  // the pairs of one radial tile read the same orbitals: batch entry fastest
+  const int bz = t % J.nbatch, bx = t / J.nbatch;
+  const TransformBatch bt = J.batch[bz];
+  const int K = J.K, C = J.C, nr = J.nr, KS = J.KS, MT = J.MT, KR = 4 * KS;
+  const int r0 = bx * R, tid = threadIdx.x;
+  const int rl = tid % R, r = r0 + rl;
   const bool row_ok = r < bt.rows;
-  const AR* __restrict__ M;
-  if constexpr (std::is_same<AR, float>::value) M = matsf + (size_t)bt.mat * K * Cp;
-  else M = mats + (size_t)bt.mat * K * Cp;
-  const AR* __restrict__ Mc = M + c0 + (lane & 15);
-  V4 dre[CT], dim[CT];
+  if constexpr (AN) {
+    const int KH = (K + 1) >> 1;
+    constexpr int U = PAIR ? 2 : 4;
+    const TI* __restrict__ x0 = in + (size_t)bt.in0 + r;
+    const TI* __restrict__ x1 = in + (size_t)bt.in1 + r;
+    for (int kb = tid / R; kb < KR; kb += KPP * U) {
+      TI xa[U], xb[U], ya[U], yb[U];
 #pragma unroll
-  for (int q = 0; q < CT; ++q) {
-    dre[q] = V4{0, 0, 0, 0};
-    dim[q] = V4{0, 0, 0, 0};
-  }
-  const int nks = (K + 3) >> 2;  // contraction steps, U per load batch
-  for (int s0 = 0; s0 < nks; s0 += U) {
-    AR a[U][CT];
-    A2 x[U];
+      for (int u = 0; u < U; ++u) {
+        const int k = kb + u * KPP;
+        const bool ok = row_ok && k < KH;
+        const size_t ga = (size_t)k * nr, gb = (size_t)(K - 1 - k) * nr;
+        xa[u] = ok ? x0[ga] : TI{};
+        xb[u] = ok ? x0[gb] : TI{};
+        if constexpr (PAIR) {
+          ya[u] = ok ? x1[ga] : TI{};
+          yb[u] = ok ? x1[gb] : TI{};
+        }
+      }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = 4 * (s0 + u) + kq;
-      const bool kok = k < K;
+      for (int u = 0; u < U; ++u) {
+        const int k = kb + u * KPP;
+        if (k >= KR) break;
+        A2 va = cto<A2>(xa[u]), vb = cto<A2>(xb[u]);
+        if constexpr (PAIR) {
+          va = cmulc(va, cto<A2>(ya[u]));
+          vb = cmulc(vb, cto<A2>(yb[u]));
+        }
+        const bool mid = 2 * k + 1 == K;
+        *reinterpret_cast<A2*>(sB + (size_t)k * NC + 2 * rl) = mid ? va : cadd(va, vb);
+        *reinterpret_cast<A2*>(sB + (size_t)(KR + k) * NC + 2 * rl) = mid ? va : csub(va, vb);
+      }
+    }
+  } else {
+    constexpr int U = 4;
+    const TI* __restrict__ x0 = in + (size_t)bt.in0 + r;
+    for (int lb = tid / R; lb < 2 * KR; lb += KPP * U) {
+      TI xv[U];
 #pragma unroll
-      for (int q = 0; q < CT; ++q) a[u][q] = (kok && q < nct) ? Mc[(size_t)k * Cp + 16 * q] : AR(0);
-      x[u] = cz<A2>();
-      if (kok && row_ok) {
-        const size_t g = (size_t)k * nr + r;
-        const TI xv = in[(size_t)bt.in0 + g];
-        x[u] = cto<A2>(xv);
+      for (int u = 0; u < U; ++u) {
+        const int l = lb + u * KPP;
+        xv[u] = (row_ok && l < K) ? x0[(size_t)l * nr] : TI{};
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int l = lb + u * KPP;
+        if (l >= 2 * KR) break;
+        const int cls = (l + bt.odd) & 1;
+        *reinterpret_cast<A2*>(sB + (size_t)(cls * KR + (l >> 1)) * NC + 2 * rl) = cto<A2>(xv[u]);
         if constexpr (std::is_same<TI, double2>::value)
-          if (copy != nullptr && by == 0) copy[(size_t)bt.in0 + g] = xv;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int q = 0; q < CT; ++q) {
-        dre[q] = MF::run(a[u][q], x[u].x, dre[q]);
-        dim[q] = MF::run(a[u][q], x[u].y, dim[q]);
-      }
-  }
-  if (row_ok) {
-#pragma unroll
-    for (int q = 0; q < CT; ++q) {
-      if (q >= nct) break;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int c = c0 + 16 * q + MF::row(lane, v);
-        A2 o;
-        o.x = dre[q][v];
-        o.y = dim[q][v];
-        if (c < C) out[(size_t)bt.out + (size_t)c * nr + r] = cto<TO>(o);
+          if (J.copy != nullptr && row_ok && l < K) J.copy[(size_t)bt.in0 + (size_t)l * nr + r] = xv[u];
       }
     }
   }
+  __syncthreads();
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const AR* __restrict__ pk = static_cast<const AR*>(J.pk) + (size_t)bt.mat * 2 * KS * MT * 64 + lane;
+  const AR* bl = sB + (size_t)(lane >> 4) * NC + (lane & 15);
+  SO* __restrict__ os = reinterpret_cast<SO*>(static_cast<TO*>(J.out) + (size_t)bt.out);
+  const int cr = (lane & 15) >> 1, comp = lane & 1;
+  // JT row tiles of 8 per item: a matrix operand loaded once serves them all
+  auto items = [&](auto jt) {
+    constexpr int JT = decltype(jt)::value;
+    const int nj = NT / JT;
+    if constexpr (AN) {
+      for (int it = wave; it < 2 * MT * nj; it += 4) {
+        const int cls = it & 1, mt = (it >> 1) % MT, j0 = (it >> 1) / MT * JT;
+        V4 d[JT];
+#pragma unroll
+        for (int j = 0; j < JT; ++j) d[j] = V4{0, 0, 0, 0};
+        const AR* __restrict__ ap = pk + ((size_t)cls * KS * MT + mt) * 64;
+        const AR* bp = bl + (size_t)cls * KR * NC + 16 * j0;
+        for (int k0 = 0; k0 < KS; k0 += 4) {
+          AR a[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) a[u] = ap[(size_t)(k0 + u) * MT * 64];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < JT; ++j) d[j] = MF::run(a[u], bp[(k0 + u) * 4 * NC + 16 * j], d[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+          const int rr = r0 + 8 * (j0 + j) + cr;
+          if (rr >= bt.rows) continue;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int c = 2 * (16 * mt + MF::row(lane, v)) + ((cls + bt.odd) & 1);
+            if (c < C) os[2 * ((size_t)c * nr + rr) + comp] = (SO)d[j][v];
+          }
+        }
+      }
+    } else {
+      const int CH = (C + 1) >> 1;
+      for (int it = wave; it < MT * nj; it += 4) {
+        const int mt = it % MT, j0 = it / MT * JT;
+        V4 de[JT], dd[JT];
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+          de[j] = V4{0, 0, 0, 0};
+          dd[j] = V4{0, 0, 0, 0};
+        }
+        const AR* __restrict__ ap = pk + (size_t)mt * 64;
+        const AR* bp = bl + 16 * j0;
+        for (int k0 = 0; k0 < KS; k0 += 4) {
+          AR ae[4], ao[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            ae[u] = ap[(size_t)(k0 + u) * MT * 64];
+            ao[u] = ap[(size_t)(KS + k0 + u) * MT * 64];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < JT; ++j) {
+              de[j] = MF::run(ae[u], bp[(k0 + u) * 4 * NC + 16 * j], de[j]);
+              dd[j] = MF::run(ao[u], bp[(KR + 4 * (k0 + u)) * NC + 16 * j], dd[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+          const int rr = r0 + 8 * (j0 + j) + cr;
+          if (rr >= bt.rows) continue;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int c = 16 * mt + MF::row(lane, v);
+            if (c >= CH) continue;
+            os[2 * ((size_t)c * nr + rr) + comp] = (SO)(de[j][v] + dd[j][v]);
+            if (C - 1 - c != c) os[2 * ((size_t)(C - 1 - c) * nr + rr) + comp] = (SO)(de[j][v] - dd[j][v]);
+          }
+        }
+      }
+    }
+  };
+  if ((AN ? 2 : 1) * MT >= 4) items(std::integral_constant<int, NT>{});
+  else items(std::integral_constant<int, 1>{});
 }
 
-template <int CT, int U, class TI, class TO>
-__global__ void __launch_bounds__(256) k_transform_mfma_w(const TI* __restrict__ in, TO* __restrict__ out,
-                                                          const double* __restrict__ mats,
-                                                          const float* __restrict__ matsf,
-                                                          const TransformBatch* __restrict__ batch, int nr, int K,
-                                                          int C, int Cp, double2* __restrict__ copy, int nx, int ny,
-                                                          int ntile, const FcPhaseJob fc) {
-  transform_mfma_w_body<CT, U, TI, TO>(in, out, mats, matsf, batch, nr, K, C, Cp, copy, nx, ny, ntile, fc, hw_blk());
+template <bool AN, bool PAIR, int NT, class TI, class TO>
+__global__ void __launch_bounds__(256) k_legendre(const LegendreJob J) {
+  legendre_body<AN, PAIR, NT, TI, TO>(J, hw_blk());
 }
 
 // ---------------------------------------------------------------------------
@@ -1519,53 +1494,51 @@ constexpr int type_code() {
                                           : (std::is_same<TO, float2>::value ? 2 : 3);
 }
 
-static void tvar_shape(int tvar, int& CT, int& U) {
-  static const int t[6][2] = {{4, 4}, {2, 4}, {4, 8}, {8, 4}, {8, 2}, {2, 8}};
-  const int v = tvar >= 0 && tvar < 6 ? tvar : 0;
-  CT = t[v][0];
-  U = t[v][1];
-}
-
 template <class T>
 static void launch_fc_phase(const FcPhaseJob& j, hipStream_t s) {
   hipLaunchKernelGGL((k_fc_phase<T>), dim3((j.nr + 255) / 256, j.nlat), dim3(256), 0, s, j);
 }
 
-constexpr long long kMfmaMinWaves = 1200;  // wavefronts of the MFMA form below which the vector form runs
+// row tiles of 8 per block: 2 (tvar 1) or 4 while the staged input stays
+// within 40 KB of LDS, so that three or more blocks share a CU; the longest
+// contractions take fewer
+static int legendre_nt(int tvar, int KS, size_t rsz) {
+  int nt = tvar == 0 ? 4 : 2;
+  while (nt > 1 && (size_t)8 * KS * 16 * nt * rsz > 40 * 1024) nt /= 2;
+  return nt;
+}
 
 template <class TI, class TO>
-void launch_transform_t(int mode, const TI* in, TO* out, const double* mats, const float* matsf,
-                        const TransformBatch* batch, int nbatch, int nr, int K, int C, int Cp, double2* copy,
-                        hipStream_t s, int path, const FcPhaseJob* fc, int tvar) {
+void launch_transform_t(int mode, const TI* in, TO* out, const LegendreMats& M, const TransformBatch* batch, int nbatch,
+                        int nr, double2* copy, hipStream_t s, int path, const FcPhaseJob* fc, int tvar) {
+  constexpr bool F32 = std::is_same<TI, float2>::value && std::is_same<TO, float2>::value;
+  const int K = M.K, C = M.C, Cp = pad_cols(C);
+  LegendreJob J{};
+  J.in = in; J.out = out; J.pk = F32 ? static_cast<const void*>(M.pkf) : static_cast<const void*>(M.pk);
+  J.batch = batch; J.nr = nr; J.K = K; J.C = C; J.nbatch = nbatch;
+  J.KS = legendre_steps(K); J.MT = legendre_tiles(C);
+  J.copy = mode == 0 ? copy : nullptr;
+  const int nt = legendre_nt(tvar, J.KS, F32 ? 4 : 8);
+  J.ntile = (nr + 8 * nt - 1) / (8 * nt) * nbatch;
+  const size_t lds = (size_t)8 * J.KS * 16 * nt * (F32 ? 4 : 8);
   if (active_recorder()) {
-    // batched form: the matrix-core kernels for every member (the same bits
-    // as the member's own matrix-core launch), 256 threads
+    // batched form: the matrix-core kernel for every member
     if (fc != nullptr) return record_unsupported("the frozen-core phase job");
-    TransformRec r;
+    LegendreJob r;
     std::memset(&r, 0, sizeof r);
-    r.in = in; r.out = out; r.mats = mats; r.matsf = matsf; r.batch = batch;
-    r.nr = nr; r.K = K; r.C = C; r.Cp = Cp; r.copy = mode == 0 ? copy : nullptr;
-    const int ct = (C + 15) / 16;
-    if (mode == 0) {
-      int CT, U;
-      tvar_shape(tvar, CT, U);
-      r.nx = (nr + 63) / 64; r.ny = (ct + CT - 1) / CT; r.ntile = r.nx * r.ny * nbatch;
-      const int var[4] = {CT, U, type_code<TI, TO>(), 0};
-      record_launch(kRecTransformW, var, dim3(r.ntile), 256, 0, r);
-    } else {
-      r.nx = (nr + 15) / 16; r.ny = (ct + 3) / 4; r.ntile = r.nx * r.ny * nbatch;
-      const int var[4] = {1, type_code<TI, TO>(), 0, 0};
-      record_launch(kRecTransformM, var, dim3(r.ntile), 256, 0, r);
-    }
+    r.in = J.in; r.out = J.out; r.pk = J.pk; r.batch = J.batch; r.copy = J.copy;
+    r.nr = J.nr; r.K = J.K; r.C = J.C; r.KS = J.KS; r.MT = J.MT; r.nbatch = J.nbatch;
+    const int rnt = tvar == 0 ? 2 : 1;  // one shape for members of any lmax
+    r.ntile = (nr + 8 * rnt - 1) / (8 * rnt) * nbatch;
+    const int var[4] = {(M.analysis ? 1 : 0) + (mode == 1 ? 2 : 0), rnt, type_code<TI, TO>(), 0};
+    record_launch(kRecLegendre, var, dim3(r.ntile), 256, (size_t)8 * J.KS * 16 * rnt * (F32 ? 4 : 8), r);
     return;
   }
-  // matrix cores (16 radial rows per block, one wavefront per 16 columns)
-  // when that gives enough wavefronts to fill the chip and at least three
-  // column tiles share each input load; otherwise the vector form, whose
-  // contraction split keeps short grids busy
-  const int ct = (C + 15) / 16;
-  const int wpb = std::min(4, ct);
-  const bool mfma = ct >= 3 && (long long)((nr + 15) / 16) * nbatch * ct >= kMfmaMinWaves;
+  // the matrix cores from 16 columns on; below, the vector form (whole hprods
+  // of 1-9 orbitals on 240-2400 points: lmax1 7 in length gauge 102 us by the
+  // vector form against 117, lmax1 31 378 against 414 (9 orbitals), lmax1 63
+  // 757 against 974; the rest within 5 %)
+  const bool mfma = C >= 16;
   if (path == 1 || (path == 0 && !mfma)) {
     const int rt = (nr + 63) / 64;
     // 8 columns per wavefront; split the contraction over 2 or 4 wavefronts
@@ -1575,58 +1548,36 @@ void launch_transform_t(int mode, const TI* in, TO* out, const double* mats, con
     while (ks < 4 && rt * ((C + 8 * (4 / ks) - 1) / (8 * (4 / ks))) * nbatch < 800) ks *= 2;
     const int cols = 8 * (4 / ks);
     dim3 grid(rt, (C + cols - 1) / cols, nbatch);
-    if (mode == 0) transform_variant<0>(ks, grid, s, in, out, mats, matsf, batch, nr, K, C, Cp, copy);
-    else transform_variant<1>(ks, grid, s, in, out, mats, matsf, batch, nr, K, C, Cp, nullptr);
+    if (mode == 0) transform_variant<0>(ks, grid, s, in, out, M.m, M.mf, batch, nr, K, C, Cp, copy);
+    else transform_variant<1>(ks, grid, s, in, out, M.m, M.mf, batch, nr, K, C, Cp, nullptr);
     if (fc != nullptr) launch_fc_phase<TO>(*fc, s);
     return;
   }
-  const FcPhaseJob fj = fc != nullptr ? *fc : FcPhaseJob{};
-  if (ct >= 2 && mode == 0) {
-    // register-blocked form: 64 rows x 16 CT columns per block, CT column
-    // tiles per wavefront, U contraction steps per load batch (for the pair
-    // products, mode 1, the form below, which forms them once per block in
-    // LDS, measured faster)
-    const int nfcb = fc != nullptr ? ((fc->nr + 255) / 256) * fc->nlat : 0;
-    auto go = [&](auto kern, int CT) {
-      const int nx = (nr + 63) / 64, ny = (ct + CT - 1) / CT, ntile = nx * ny * nbatch;
-      hipLaunchKernelGGL(kern, dim3(ntile + nfcb), dim3(256), 0, s, in, out, mats, matsf, batch, nr, K, C, Cp, copy,
-                         nx, ny, ntile, fj);
-    };
-    switch (tvar) {
-      case 1: go(k_transform_mfma_w<2, 4, TI, TO>, 2); break;
-      case 2: go(k_transform_mfma_w<4, 8, TI, TO>, 4); break;
-      case 3: go(k_transform_mfma_w<8, 4, TI, TO>, 8); break;
-      case 4: go(k_transform_mfma_w<8, 2, TI, TO>, 8); break;
-      case 5: go(k_transform_mfma_w<2, 8, TI, TO>, 2); break;
-      default: go(k_transform_mfma_w<4, 4, TI, TO>, 4); break;
-    }
-    return;
-  }
-  const int nx = (nr + 15) / 16, ny = (ct + wpb - 1) / wpb, ntile = nx * ny * nbatch;
-  const int nfcb = fc != nullptr ? ((fc->nr + 64 * wpb - 1) / (64 * wpb)) * fc->nlat : 0;
-  if (mode == 0)
-    hipLaunchKernelGGL((k_transform_mfma<0, TI, TO>), dim3(ntile + nfcb), dim3(64 * wpb), 0, s, in, out, mats, matsf,
-                       batch, nr, K, C, Cp, copy, nx, ny, ntile, fj);
-  else
-    hipLaunchKernelGGL((k_transform_mfma<1, TI, TO>), dim3(ntile + nfcb), dim3(64 * wpb), 0, s, in, out, mats, matsf,
-                       batch, nr, K, C, Cp, nullptr, nx, ny, ntile, fj);
+  if (fc != nullptr) J.fc = *fc;
+  const int nfcb = fc != nullptr ? ((fc->nr + 255) / 256) * fc->nlat : 0;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(J.ntile + nfcb), dim3(256), lds, s, J); };
+  auto by_nt = [&](auto an, auto pair) {
+    constexpr bool AN = decltype(an)::value, PAIR = decltype(pair)::value;
+    if (nt == 4) go(k_legendre<AN, PAIR, 4, TI, TO>);
+    else if (nt == 2) go(k_legendre<AN, PAIR, 2, TI, TO>);
+    else go(k_legendre<AN, PAIR, 1, TI, TO>);
+  };
+  if (mode == 1) by_nt(std::true_type{}, std::true_type{});
+  else if (M.analysis) by_nt(std::true_type{}, std::false_type{});
+  else by_nt(std::false_type{}, std::false_type{});
 }
-template void launch_transform_t<double2, float2>(int, const double2*, float2*, const double*, const float*,
-                                                  const TransformBatch*, int, int, int, int, int, double2*,
-                                                  hipStream_t, int, const FcPhaseJob*, int);
-template void launch_transform_t<float2, float2>(int, const float2*, float2*, const double*, const float*,
-                                                 const TransformBatch*, int, int, int, int, int, double2*,
-                                                 hipStream_t, int, const FcPhaseJob*, int);
-template void launch_transform_t<float2, double2>(int, const float2*, double2*, const double*, const float*,
-                                                  const TransformBatch*, int, int, int, int, int, double2*,
-                                                  hipStream_t, int, const FcPhaseJob*, int);
-
-void launch_transform(int mode, const double2* in, double2* out, const double* mats, const TransformBatch* batch,
-                      int nbatch, int nr, int K, int C, int Cp, double2* copy, hipStream_t s, int path,
-                      const FcPhaseJob* fc, int tvar) {
-  launch_transform_t<double2, double2>(mode, in, out, mats, nullptr, batch, nbatch, nr, K, C, Cp, copy, s, path, fc,
-                                       tvar);
-}
+template void launch_transform_t<double2, double2>(int, const double2*, double2*, const LegendreMats&,
+                                                   const TransformBatch*, int, int, double2*, hipStream_t, int,
+                                                   const FcPhaseJob*, int);
+template void launch_transform_t<double2, float2>(int, const double2*, float2*, const LegendreMats&,
+                                                  const TransformBatch*, int, int, double2*, hipStream_t, int,
+                                                  const FcPhaseJob*, int);
+template void launch_transform_t<float2, float2>(int, const float2*, float2*, const LegendreMats&,
+                                                 const TransformBatch*, int, int, double2*, hipStream_t, int,
+                                                 const FcPhaseJob*, int);
+template void launch_transform_t<float2, double2>(int, const float2*, double2*, const LegendreMats&,
+                                                  const TransformBatch*, int, int, double2*, hipStream_t, int,
+                                                  const FcPhaseJob*, int);
 
 // shape: 0 = 3 elements per block (one wavefront), 1 = 6 (128 threads),
 // 2 = 12 (256 threads); lc = l values per block
@@ -2701,8 +2652,7 @@ Recorder*& active_recorder() {
 
 size_t rec_size(int kind) {
   switch (kind) {
-    case kRecTransformW:
-    case kRecTransformM: return sizeof(TransformRec);
+    case kRecLegendre: return sizeof(LegendreJob);
     case kRecOneBody: return sizeof(OneBodyRec);
     case kRecPoissonBridge:
     case kRecPoissonInterior: return sizeof(PoissonRec);
@@ -2720,27 +2670,13 @@ size_t rec_size(int kind) {
   }
 }
 
-template <int CT, int U, class TI, class TO>
-__global__ void __launch_bounds__(256) k_transform_mfma_w_batch(const TransformRec* __restrict__ recs,
-                                                                const BatchMap map) {
-  __shared__ __align__(16) unsigned char raw[sizeof(TransformRec)];
+template <bool AN, bool PAIR, int NT, class TI, class TO>
+__global__ void __launch_bounds__(256) k_legendre_batch(const LegendreJob* __restrict__ recs, const BatchMap map) {
+  __shared__ __align__(16) unsigned char raw[sizeof(LegendreJob)];
   int have = -1;
   batch_walk(map, NoSkip(), [&](int m, const Blk& bk) {
-    const TransformRec& r = stage_rec(recs, m, raw, have);
-    transform_mfma_w_body<CT, U, TI, TO>(static_cast<const TI*>(r.in), static_cast<TO*>(r.out), r.mats, r.matsf,
-                                         r.batch, r.nr, r.K, r.C, r.Cp, r.copy, r.nx, r.ny, r.ntile, r.fc, bk);
-  });
-}
-
-template <int MODE, class TI, class TO>
-__global__ void __launch_bounds__(256) k_transform_mfma_batch(const TransformRec* __restrict__ recs,
-                                                              const BatchMap map) {
-  __shared__ __align__(16) unsigned char raw[sizeof(TransformRec)];
-  int have = -1;
-  batch_walk(map, NoSkip(), [&](int m, const Blk& bk) {
-    const TransformRec& r = stage_rec(recs, m, raw, have);
-    transform_mfma_body<MODE, TI, TO>(static_cast<const TI*>(r.in), static_cast<TO*>(r.out), r.mats, r.matsf, r.batch,
-                                      r.nr, r.K, r.C, r.Cp, r.copy, r.nx, r.ny, r.ntile, r.fc, bk);
+    const LegendreJob& r = stage_rec(recs, m, raw, have);
+    legendre_body<AN, PAIR, NT, TI, TO>(r, bk);
   });
 }
 
@@ -2961,26 +2897,31 @@ bool launch_batch_kernels(const LaunchRec& p, const void* recs, const BatchMap& 
     if (!dry) hipLaunchKernelGGL((K), g, b, lds, s, static_cast<const R*>(recs), map); \
   } while (0)
   switch (p.kind) {
-    case kRecTransformW: {
+    case kRecLegendre: {
       if (p.block != 256) return false;
-      switch (p.var[0] * 100 + p.var[1] * 10 + p.var[2]) {
-        case 240: TD1C_BATCH((k_transform_mfma_w_batch<2, 4, double2, double2>), TransformRec); return true;
-        case 241: TD1C_BATCH((k_transform_mfma_w_batch<2, 4, double2, float2>), TransformRec); return true;
-        case 242: TD1C_BATCH((k_transform_mfma_w_batch<2, 4, float2, float2>), TransformRec); return true;
-        case 243: TD1C_BATCH((k_transform_mfma_w_batch<2, 4, float2, double2>), TransformRec); return true;
-        case 440: TD1C_BATCH((k_transform_mfma_w_batch<4, 4, double2, double2>), TransformRec); return true;
-        case 441: TD1C_BATCH((k_transform_mfma_w_batch<4, 4, double2, float2>), TransformRec); return true;
-        case 442: TD1C_BATCH((k_transform_mfma_w_batch<4, 4, float2, float2>), TransformRec); return true;
-        case 443: TD1C_BATCH((k_transform_mfma_w_batch<4, 4, float2, double2>), TransformRec); return true;
+      auto by_nt = [&](auto an, auto pair, auto ti, auto to) {
+        constexpr bool AN = decltype(an)::value, PAIR = decltype(pair)::value;
+        using TI = decltype(ti);
+        using TO = decltype(to);
+        if (p.var[1] == 1) TD1C_BATCH((k_legendre_batch<AN, PAIR, 1, TI, TO>), LegendreJob);
+        else if (p.var[1] == 2) TD1C_BATCH((k_legendre_batch<AN, PAIR, 2, TI, TO>), LegendreJob);
+        else return false;
+        return true;
+      };
+      const double2 d{};
+      const float2 f{};
+      const std::false_type n{};
+      const std::true_type y{};
+      switch (p.var[0] * 10 + p.var[2]) {  // direction (0 l -> theta, 1 theta -> l, 3 pair products), types
+        case 0: return by_nt(n, n, d, d);
+        case 1: return by_nt(n, n, d, f);
+        case 2: return by_nt(n, n, f, f);
+        case 10: return by_nt(y, n, d, d);
+        case 13: return by_nt(y, n, f, d);
+        case 30: return by_nt(y, y, d, d);
+        case 32: return by_nt(y, y, f, f);
         default: return false;
       }
-    }
-    case kRecTransformM: {
-      if (p.block != 256 || p.var[0] != 1) return false;
-      if (p.var[1] == 0) TD1C_BATCH((k_transform_mfma_batch<1, double2, double2>), TransformRec);
-      else if (p.var[1] == 2) TD1C_BATCH((k_transform_mfma_batch<1, float2, float2>), TransformRec);
-      else return false;
-      return true;
     }
     case kRecOneBody: {
       switch (p.var[0] * 10 + p.var[1]) {

@@ -37,6 +37,7 @@ struct TransformBatch {
   long long out;   // element offset of the output block
   int mat;         // matrix index (m + mmax)
   int rows;        // radial rows to compute (nr, or nradfc for frozen core)
+  int odd;         // |m| & 1
 };
 
 struct OneBodyArgs {
@@ -242,18 +243,40 @@ struct FcPhaseJob {
   int nr, nradfc, nlat, nfc;
 };
 
-// path: 0 by grid size, 1 the vector form, 2 the matrix-core (MFMA) form
-// tvar: launch shape of the register-blocked matrix-core form (0..5, same bits)
-void launch_transform(int mode, const double2* in, double2* out, const double* mats, const TransformBatch* batch,
-                      int nbatch, int nr, int K, int C, int Cp, double2* copy, hipStream_t s, int path = 0,
-                      const FcPhaseJob* fc = nullptr, int tvar = 0);
+// One direction of the Legendre transforms: the K x C matrices of every m,
+// plain ([m][K][pad_cols(C)], for the vector form) and packed for the
+// matrix-core form: per m and parity class, step ks and column tile mt the 64
+// lane values of an MFMA A operand, over the half of the theta points
+// (theta -> l: k the first (K+1)/2 points, columns l of the class; l -> theta:
+// k the l of the class, columns the first (C+1)/2 points).  The l of class c
+// are 2 i + ((c + m) & 1).  mf, pkf: the same in FP32, used when both sides
+// are complex64.
+struct LegendreMats {
+  int analysis;  // 1: theta -> l
+  int K, C;
+  const double *m, *pk;
+  const float *mf, *pkf;
+};
+inline int legendre_steps(int K) { return ((K + 1) / 2 + 15) / 16 * 4; }  // whole load batches of 4, zeros beyond K
+inline int legendre_tiles(int C) { return ((C + 1) / 2 + 15) / 16; }
+// one launch of the matrix-core form
+struct LegendreJob {
+  const void* in;
+  void* out;
+  const void* pk;
+  const TransformBatch* batch;
+  double2* copy;  // l -> theta: the input copied here as it is read (may be null)
+  int nr, K, C, KS, MT, nbatch, ntile, pad;
+  FcPhaseJob fc;
+};
 inline int pad_cols(int C) { return (C + 31) / 32 * 32; }
-// the same transform with complex64 on either side (matsf: the matrices in
-// FP32, used when both sides are complex64)
+// mode 0: plain input; 1: pair products (theta -> l).  path: 0 by grid size,
+// 1 the vector form, 2 the matrix-core (MFMA) form; tvar: rows per block of
+// the matrix-core form (0: 32, else 16; same bits)
 template <class TI, class TO>
-void launch_transform_t(int mode, const TI* in, TO* out, const double* mats, const float* matsf,
-                        const TransformBatch* batch, int nbatch, int nr, int K, int C, int Cp, double2* copy,
-                        hipStream_t s, int path = 0, const FcPhaseJob* fc = nullptr, int tvar = 0);
+void launch_transform_t(int mode, const TI* in, TO* out, const LegendreMats& M, const TransformBatch* batch, int nbatch,
+                        int nr, double2* copy, hipStream_t s, int path = 0, const FcPhaseJob* fc = nullptr,
+                        int tvar = 1);
 void launch_onebody(const double2* orb, double2* h01, const OneBodyArgs& a, hipStream_t s);
 // shape 0/1/2: 3/6/12 elements per block; lc: l values per block (any
 // shape gives the same bits; the autotuner picks one per problem)
@@ -443,8 +466,7 @@ __device__ __forceinline__ const R& stage_rec(const R* __restrict__ recs, int m,
 }
 
 enum RecKind {
-  kRecTransformW = 1,   // var: CT, U, type code
-  kRecTransformM,       // var: MODE, type code (256 threads)
+  kRecLegendre = 1,     // var: direction (1 theta -> l) + 2 (pair products), row tiles, type code
   kRecOneBody,          // var: GE, CN
   kRecPoissonBridge,    // var: type code (LDS form, ndvr = 20)
   kRecPoissonInterior,  // var: type code
@@ -460,17 +482,6 @@ enum RecKind {
   kRecCnCheck,
 };
 // type codes of (input, output): 0 (c128, c128), 1 (c128, c64), 2 (c64, c64), 3 (c64, c128)
-struct TransformRec {
-  const void* in;
-  void* out;
-  const double* mats;
-  const float* matsf;
-  const TransformBatch* batch;
-  int nr, K, C, Cp;
-  double2* copy;
-  int nx, ny, ntile;
-  FcPhaseJob fc;
-};
 // In a batch, the terms of the half-step series share one word: the check
 // of term k stores k when some member has not converged, and a launch of
 // term k > 1 (right-hand side, bridge, interior, check) runs only when the

@@ -1,0 +1,41 @@
+"""Kernels at the edges of their tiles, against the oracle: relative 2-norm of
+the derivative, 1e-11 in FP64 (the L = 0 Poisson operator's conditioning) and
+1e-5 with the complex64 mean field, as in test_gpu_parity."""
+import numpy as np
+import pytest
+
+import td1c_amd
+from oracle.oracle import Oracle
+from td1c_amd.abi import Problem
+from tests import cases as C
+
+pytestmark = pytest.mark.gpu
+
+
+def hprod_error(prob, lf, path=0):
+    import torch
+
+    o = Oracle(prob)
+    w = C.wfn_for(prob, o.lcic)
+    o.set_wfn0(w)
+    ref = o.htot(1.0, lf, w)
+    hp = td1c_amd.HProd(prob)
+    hp.set_transform_path(path)
+    hp.set_wfn0(w)
+    out = hp.htot(1.0, lf, hp.to_device(w))
+    torch.cuda.synchronize()
+    return np.linalg.norm(out.cpu().numpy() - ref) / np.linalg.norm(ref)
+
+
+# the matrix-core Legendre transform: column tiles of 16 per parity class
+# (lmax 14..17, 31..33 around one and two tiles), odd and even numbers of
+# theta points (the middle point), orders m whose classes swap, rows that end
+# inside a tile of 8 or 16 (nfe * 20 - 1 points)
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("lmax1,lmax2,nlat,mval", [
+    (1, 2, 0, [0, 1]), (6, 13, 0, [0, 1]), (7, 14, 16, [0, 1]), (15, 31, 0, [0, -1]), (16, 30, 33, [1, -1]),
+    (17, 33, 0, [0, 0]), (31, 63, 0, [0, 1]), (32, 64, 66, [0, 0])])
+def test_legendre_tiles(gpu_lib, lmax1, lmax2, nlat, mval, precision):
+    prob = Problem(nfe=3, ndvr=20, rmax=9.0, lmax1=lmax1, lmax2=lmax2, nlat=nlat, znuc=4.0, ndcore=2, nel_alpha=2,
+                   nel_beta=2, mval=mval, precision=precision)
+    assert hprod_error(prob, C.LF_LEN, path=2) < (1e-5 if precision else 1e-11)
