@@ -118,7 +118,7 @@ struct td1c_ctx {
   DevBuf<double2> gram_partial, gram_partial_p, lprod, pprod;
   DevBuf<int> mapH, mapG, mapV, mapF, map2e;
   // island
-  DevBuf<double2> den1, den2, rden, rrden, int1e, int2e, xmat, dcic, ci_work, mfc, dip_part, ovlp;
+  DevBuf<double2> den1, den2, rden, rrden, int1e, int2e, xmat, dcic, ci_work, ci_gram, ci_hp, mfc, dip_part, ovlp;
   DevBuf<double> ene;
   DevBuf<int> det_of, exA, sgA, exB, sgB;
   double ene_fcore = 0.0;
@@ -232,7 +232,7 @@ struct td1c_ctx {
                             &cnG, &cnWl, &cnWr, &cnPa, &cnPg, &cnBinv, &cn_x, &cn_y, &vfc_tab, &gfc_g, &gfc_l,
                             &dipfc_part,
                             &gram_partial, &gram_partial_p, &lprod, &pprod, &den1, &den2, &rden, &rrden, &int1e, &int2e, &xmat,
-                            &dcic, &ci_work, &mfc, &dip_part, &ovlp, &rk_w0, &rk_t, &rk_k};
+                            &dcic, &ci_work, &ci_gram, &ci_hp, &mfc, &dip_part, &ovlp, &rk_w0, &rk_t, &rk_k};
     for (auto* b : z) b->release();
     DevBuf<int>* i[] = {&mval, &lval, &pair_m, &pj, &pi, &ptype, &emap, &mapH, &mapG, &mapV, &mapF, &map2e, &cn_flag,
                         &det_of, &exA, &sgA, &exB, &sgB};
@@ -700,6 +700,8 @@ int build_device(td1c_ctx* c) {
   HIP_TRY(c->dip3_tmp.alloc(3));
   HIP_TRY(c->ovlp.alloc((size_t)S.nfun * S.nfun));
   HIP_TRY(c->ci_work.alloc(std::max<size_t>(1, ((size_t)2 * S.nact * S.nact + 2) * nfull)));
+  HIP_TRY(c->ci_gram.alloc((size_t)(na * na + 1) * (na * na + 1)));
+  HIP_TRY(c->ci_hp.alloc((size_t)na * na));
   HIP_TRY(c->det_of.upload(flat_or_one(S.det_of)));
   HIP_TRY(c->exA.upload(flat_or_one(S.exA)));
   HIP_TRY(c->sgA.upload(flat_or_one(S.sgA)));
@@ -738,7 +740,7 @@ IslandArgs island_args(td1c_ctx* c, const double2* cic, double dtime) {
   a.throcc1 = S.throcc1; a.throcc2 = S.throcc2; a.dtime = dtime;
   a.nstr_a = S.nstr_a; a.nstr_b = S.nstr_b;
   a.det_of = c->det_of.p; a.exA = c->exA.p; a.sgA = c->sgA.p; a.exB = c->exB.p; a.sgB = c->sgB.p;
-  a.cic = cic; a.ci_work = c->ci_work.p;
+  a.cic = cic; a.ci_work = c->ci_work.p; a.ci_gram = c->ci_gram.p; a.ci_hp = c->ci_hp.p;
   a.den1 = c->den1.p; a.den2 = c->den2.p; a.rden = c->rden.p; a.rrden = c->rrden.p;
   a.lprod = c->lprod.p;
   a.lpart = c->gram_partial.p;

@@ -199,8 +199,10 @@ struct IslandArgs {
   const double2* cic;
   double2* ci_work;       // (2 nact^2 + 2) * nstr_a * nstr_b; holds D_pq = E_pq C between the stages
   // dynamic LDS plan (island_lds_plan): CI work and string tables in LDS,
-  // int2e in LDS at byte offset ci_lds_off
+  // int2e in LDS at byte offset ci_lds_off; without room for the CI work
+  // (ci_lds = 0, active orbitals) the CI parts run as launches over the chip
   int ci_lds, i2_lds;
+  double2 *ci_gram, *ci_hp;  // [(nact^2 + 1)^2] overlaps of the E_pq C and C; [nact^2] h'_pq
   size_t ci_lds_off, lds_bytes;
   // stage A outputs
   double2 *den1, *den2, *rden, *rrden;
