@@ -473,7 +473,6 @@ enum RecKind {
   kRecPoissonBridge,    // var: type code (LDS form, ndvr = 20)
   kRecPoissonInterior,  // var: type code
   kRecMfprodT,          // var: NF, type code (dynamical cores only)
-  kRecMfprod,           // var: type code
   kRecGram,             // var: TA, TB, CR, f32
   kRecDtorb,
   kRecMask,

@@ -39,3 +39,19 @@ def test_legendre_tiles(gpu_lib, lmax1, lmax2, nlat, mval, precision):
     prob = Problem(nfe=3, ndvr=20, rmax=9.0, lmax1=lmax1, lmax2=lmax2, nlat=nlat, znuc=4.0, ndcore=2, nel_alpha=2,
                    nel_beta=2, mval=mval, precision=precision)
     assert hprod_error(prob, C.LF_LEN, path=2) < (1e-5 if precision else 1e-11)
+
+
+# the register-resident mean-field kernels of each orbital partition (frozen
+# cores, dynamical cores, active orbitals), one beyond them on either side
+# (the generic kernel), and the CI launches of long CI vectors (5 and more
+# active orbitals): one determinant short of the LDS budget up to 4900
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nfc,ndc,nact,nel", [
+    (0, 5, 0, 0), (0, 12, 0, 0), (0, 0, 2, 2), (0, 0, 3, 2), (1, 0, 2, 2), (1, 0, 3, 4), (0, 1, 3, 2), (1, 1, 2, 2),
+    (1, 1, 4, 4), (0, 2, 2, 2), (0, 1, 4, 2), (0, 0, 5, 2), (0, 0, 5, 4), (1, 0, 5, 6), (0, 1, 5, 4), (1, 0, 6, 8),
+    (0, 0, 6, 2), (1, 1, 6, 2), (1, 0, 7, 2), (0, 0, 8, 8), (1, 0, 8, 2)])
+def test_partitions(gpu_lib, nfc, ndc, nact, nel, precision):
+    n = nfc + ndc + nel // 2
+    prob = Problem(nfe=3, ndvr=20, rmax=9.0, lmax1=3, lmax2=6, znuc=4.0, nfcore1=nfc, ndcore=ndc, nact=nact, nel_alpha=n,
+                   nel_beta=n, lval=[0] * (nfc + ndc + nact), igauge=1, precision=precision)
+    assert hprod_error(prob, C.LF_VEL) < (1e-5 if precision else 1e-11)
