@@ -88,8 +88,8 @@ struct td1c_ctx {
   int npair = 0, nd = 0, nbas = 0, ngrid = 0;
   int device = 0;
   // tables
-  DevBuf<double> xr, band_k, band_k0, band_p, alph, cost, mask;
-  DevBuf<double2> tdiag, tzor;
+  DevBuf<double> xr, band_p, alph, cost, mask;
+  DevBuf<double2> tzor;
   DevBuf<double> eK0, eK, eP;
   DevBuf<double> m_l2g, m_g2l, m_g2L, m_L2g;
   DevBuf<double> k_l2g, k_g2l, k_g2L, k_L2g;  // packed for the matrix cores
@@ -224,11 +224,11 @@ struct td1c_ctx {
   std::vector<std::pair<std::string, std::pair<double, int>>> timing_agg;
 
   ~td1c_ctx() {
-    DevBuf<double>* d[] = {&eK0, &eK, &eP, &xr, &band_k, &band_k0, &band_p, &alph, &cost, &mask, &m_l2g, &m_g2l, &m_g2L, &m_L2g, &k_l2g, &k_g2l, &k_g2L, &k_L2g,
+    DevBuf<double>* d[] = {&eK0, &eK, &eP, &xr, &band_p, &alph, &cost, &mask, &m_l2g, &m_g2l, &m_g2L, &m_L2g, &k_l2g, &k_g2l, &k_g2L, &k_L2g,
                            &pG, &pWl, &pWr, &pWlI, &pWrI, &pcrA, &pcrG, &pcrBinv, &pSd, &pSl, &pSu, &invr, &rpl0, &rpl1, &fac2, &fac1, &ene, &lf_dev,
                        &cn_part, &lf_cn};
     for (auto* b : d) b->release();
-    DevBuf<double2>* z[] = {&tdiag, &tzor, &lsp, &gsp, &orbg0, &rhoL, &vL, &vg, &p_xb, &p_Q, &legacy_stage,
+    DevBuf<double2>* z[] = {&tzor, &lsp, &gsp, &orbg0, &rhoL, &vL, &vg, &p_xb, &p_Q, &legacy_stage,
                             &cnG, &cnWl, &cnWr, &cnPa, &cnPg, &cnBinv, &cn_x, &cn_y, &vfc_tab, &gfc_g, &gfc_l,
                             &dipfc_part,
                             &gram_partial, &gram_partial_p, &lprod, &pprod, &den1, &den2, &rden, &rrden, &int1e, &int2e, &xmat,
@@ -426,8 +426,6 @@ int build_device(td1c_ctx* c) {
   c->npair = (int)S.pairs.size();
   HIP_TRY(hipGetDevice(&c->device));
   HIP_TRY(c->xr.upload(S.xr));
-  HIP_TRY(c->band_k.upload(S.bandT_k));
-  HIP_TRY(c->band_k0.upload(S.bandT_k0));
   HIP_TRY(c->band_p.upload(S.bandT_p));
   HIP_TRY(c->alph.upload(S.alph));
   HIP_TRY(c->cost.upload(S.cost));
@@ -437,12 +435,8 @@ int build_device(td1c_ctx* c) {
     HIP_TRY(c->mask.upload(m));
   }
   {
-    std::vector<double2> td((size_t)L1 * nr), tz((size_t)L1 * nr);
-    for (size_t q = 0; q < td.size(); ++q) {
-      td[q] = make_double2(S.tdiag[2 * q], S.tdiag[2 * q + 1]);
-      tz[q] = make_double2(S.tzor[2 * q], S.tzor[2 * q + 1]);
-    }
-    HIP_TRY(c->tdiag.upload(td));
+    std::vector<double2> tz((size_t)L1 * nr);
+    for (size_t q = 0; q < tz.size(); ++q) tz[q] = make_double2(S.tzor[2 * q], S.tzor[2 * q + 1]);
     HIP_TRY(c->tzor.upload(tz));
   }
   HIP_TRY(c->eK0.upload(S.eK0));
@@ -855,16 +849,10 @@ int enqueue_htotx(td1c_ctx* c, double dtime, const double* d_lf, const double2* 
   // stream needs neither before the l-space Gram products)
   enqueue_orbin_fc_l(c, s2);
   // one-body part
-  OneBodyArgs ob{};
-  ob.nr = nr; ob.L1 = L1; ob.ndvr = S.n; ob.nfcore = nfc; ob.nradfc = S.nradfc;
-  ob.mmax1 = S.mmax1; ob.igauge = S.igauge; ob.fc_full = S.iprojfc == 2;
-  ob.mval = c->mval.p; ob.band_k = c->band_k.p; ob.band_k0 = c->band_k0.p; ob.band_p = c->band_p.p;
-  ob.xr = c->xr.p; ob.alph = c->alph.p; ob.tdiag = c->tdiag.p; ob.lf = d_lf;
-  ob.f0 = 0; ob.f1 = nf;
   const OneBodyElArgs oe = onebody_el_args(c, d_lf);
   {
     TIMED_ON(s2, "onebody");
-    if (!launch_onebody_el(c->orb, c->h01, oe, s2, c->ob_shape, c->ob_lc)) launch_onebody(c->orb, c->h01, ob, s2);
+    launch_onebody_el(c->orb, c->h01, oe, s2, c->ob_shape, c->ob_lc);
   }
   HIP_TRY(hipEventRecord(c->fj[3], s2));
   bool pair_gram_done = false;
@@ -1167,7 +1155,6 @@ int autotune_onebody(td1c_ctx* c) {
   static std::mutex mu;
   static std::map<std::string, std::pair<int, int>> cache;
   const Setup& S = c->S;
-  if (S.n != 20) return 0;  // the band kernel runs for other ndvr
   const char* env = std::getenv("TD1C_AUTOTUNE");
   if (env && std::string(env) == "0") return 0;
   const std::string key = onebody_shape_key(S);
@@ -1449,14 +1436,12 @@ int td1c_set_wfn0(td1c_ctx* c, const double* wfn, const double* cic, const doubl
   }
   c->cn_dt = 0.0;
   // tmat += v2jfc (hprod_addfc_tmat)
-  std::vector<double2> td((size_t)L1 * nr), tz((size_t)L1 * nr);
+  std::vector<double2> tz((size_t)L1 * nr);
   for (int l = 0; l < L1; ++l)
     for (int i = 0; i < nr; ++i) {
       size_t q = (size_t)l * nr + i;
-      td[q] = make_double2(S.tdiag[2 * q] + v2jfc[i].x, S.tdiag[2 * q + 1] + v2jfc[i].y);
       tz[q] = make_double2(S.tzor[2 * q] + v2jfc[i].x, S.tzor[2 * q + 1] + v2jfc[i].y);
     }
-  HIP_TRY(hipMemcpy(c->tdiag.p, td.data(), td.size() * sizeof(double2), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->tzor.p, tz.data(), tz.size() * sizeof(double2), hipMemcpyHostToDevice));
   return 0;
 }
@@ -2048,8 +2033,7 @@ static CnArgs cn_args(td1c_ctx* c, const double* d_lf, double2* wfn) {
   a.nr = S.nr; a.n = S.n; a.nfe = S.nfe; a.ni = S.n - 1; a.nb = S.nfe - 1; a.K = c->cn_K; a.L1 = S.L1;
   a.nfun = S.nfun; a.nfcore = S.nfcore; a.mmax1 = S.mmax1; a.igauge = S.igauge; a.isplit = S.isplit;
   a.mval = c->mval.p;
-  a.band_k = c->band_k.p; a.band_k0 = c->band_k0.p; a.band_p = c->band_p.p; a.tdiag = c->tdiag.p;
-  a.xr = c->xr.p; a.alph = c->alph.p; a.lf = d_lf;
+  a.lf = d_lf;
   a.G = c->cnG.p; a.gstride = S.nfe; a.Wl = c->cnWl.p; a.Wr = c->cnWr.p; a.pa = c->cnPa.p; a.pg = c->cnPg.p; a.binv = c->cnBinv.p;
   a.wfn = wfn; a.x = c->cn_x.p; a.y = c->cn_y.p;
   const double q = 0.25 * c->cn_dt;
@@ -2068,7 +2052,7 @@ static CnArgs cn_args(td1c_ctx* c, const double* d_lf, double2* wfn) {
 // device to get there) and stops enqueuing once the series has converged:
 // the later terms would all return at once, and each would still cost its
 // launches.
-static int enqueue_series(td1c_ctx* c, const CnArgs& a, const OneBodyElArgs* obp, int maxcyc, hipStream_t s) {
+static int enqueue_series(td1c_ctx* c, const CnArgs& a, const OneBodyElArgs& obp, int maxcyc, hipStream_t s) {
   if (c->capturing || active_recorder()) {
     for (int k = 0; k < maxcyc; ++k) launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 1, s);
     return 0;
@@ -2092,7 +2076,7 @@ static int enqueue_series(td1c_ctx* c, const CnArgs& a, const OneBodyElArgs* obp
 // after convergence.
 static int enqueue_h1itr(td1c_ctx* c, const double* d_lf, double2* wfn, hipStream_t s) {
   const CnArgs a = cn_args(c, d_lf, wfn);
-  // the right-hand sides by the element one-body kernel (ndvr = 20): over
+  // the right-hand sides by the element one-body kernel: over
   // the dynamical orbitals, with the field of this half step
   OneBodyElArgs ob = onebody_el_args(c, d_lf);
   ob.nfun = c->S.nfun - c->S.nfcore;
@@ -2101,10 +2085,9 @@ static int enqueue_h1itr(td1c_ctx* c, const double* d_lf, double2* wfn, hipStrea
   ob.isplit = c->S.isplit;
   ob.cv = a.zfac1;
   ob.stop = a.flag;
-  const OneBodyElArgs* obp = c->S.n == 20 ? &ob : nullptr;
   TIMED("h1itr");
-  launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 0, s);
-  return enqueue_series(c, a, obp, c->cn_maxcyc, s);
+  launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, 0, s);
+  return enqueue_series(c, a, ob, c->cn_maxcyc, s);
 }
 
 static int enqueue_rk_step(td1c_ctx* c, int rk_order, double dtime, const double* d_lf, double2* wfn, int apply_mask,
@@ -2703,7 +2686,6 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
   // the field of the rational functions: cletdrb's timeh = t (etd_time_of_h
   // 0), cletdrk4's thalf = t + dt/2, clexpab's t
   const double* lfr = c->etd_scheme == 2 ? lf1 : lf0;
-  const bool ob_el = S.n == 20;
   auto cpy = [&](double2* z, const double2* x, size_t n) { launch_zaxpby(n, one, x, zero, nullptr, z, s); };
   auto clr = [&](double2* z, size_t n) { launch_zaxpby(n, zero, nullptr, zero, nullptr, z, s); };
   // y += a x
@@ -2724,7 +2706,7 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
     a.zfac1 = cv;
     a.flag = c->etd_zero.p;
     const OneBodyElArgs ob = ob_args(lf);
-    launch_cn_stage(a, ob_el ? &ob : nullptr, c->ob_shape, c->ob_lc, vonly ? 4 : 3, s);
+    launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, vonly ? 4 : 3, s);
   };
   // the numerator sum_k cn[k] (dt h1)^k of R on in (dynamical rows) into out
   auto numer = [&](const td1c_ctx::EtdRat& R, const double2* in, double2* out) {
@@ -2753,10 +2735,9 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
       OneBodyElArgs ob = ob_args(lfr);
       ob.cv = a.zfac1;
       ob.stop = a.flag;
-      const OneBodyElArgs* obp = ob_el ? &ob : nullptr;
-      launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 2, s);
+      launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, 2, s);
       if (S.isplit == 1 && S.icomp == 1)
-        if (int rc = enqueue_series(c, a, obp, c->etd_maxcyc, s)) series_err = rc;
+        if (int rc = enqueue_series(c, a, ob, c->etd_maxcyc, s)) series_err = rc;
     }
   };
   auto cmulh = [](double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
@@ -2861,9 +2842,8 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
       OneBodyElArgs ob = ob_args(lf1);
       ob.cv = a.zfac1;
       ob.stop = a.flag;
-      const OneBodyElArgs* obp = ob_el ? &ob : nullptr;
-      launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 2, s);
-      if (int rc = enqueue_series(c, a, obp, c->etd_maxcyc, s)) series_err = rc;
+      launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, 2, s);
+      if (int rc = enqueue_series(c, a, ob, c->etd_maxcyc, s)) series_err = rc;
       launch_zaxpby(so, make_double2(-1.0, 0.0), in, make_double2(2.0, 0.0), out, out, s);
     };
     const double dt = c->etd_dt;

@@ -11,8 +11,7 @@
 // of each FEDVR element are eliminated with their precomputed inverses and
 // the bridge points form a tridiagonal system solved by cyclic reduction.
 // One term of the series is four launches: the right-hand side (the
-// element one-body kernel in its Crank-Nicolson modes, or a band kernel for
-// ndvr != 20), the bridge pass (one block per orbital row), the interior
+// element one-body kernel in its Crank-Nicolson modes), the bridge pass (one block per orbital row), the interior
 // pass (one block per (l, element chunk), each element inverse read once for
 // every orbital) and the convergence test (one block); every later launch of
 // the half step returns at once after convergence.
@@ -25,92 +24,6 @@
 #include "kernels.hpp"
 
 namespace td1c {
-
-// Right-hand side, thread per (r, l, dynamical orbital):
-// mode 0: y = psi - c (T psi + V psi)   (V with isplit = 1 only;
-//         hprod_tprod_dyn + hprod_zprod_dyn / hprod_pzprod_dyn, then the
-//         zaxpy of h1itr_prop.F90:57-70)
-// mode 1: y = -c V x                    (h1itr_prop.F90:106-114)
-// mode 3: y = zfac1 (T x + V x)         (hprod_h1tot, hprod_h1tot.F90:2-53)
-__global__ void __launch_bounds__(256) k_cn_rhs(const CnArgs a, int mode) {
-  if (mode == 1 && a.flag[0]) return;
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const int l = blockIdx.y;
-  const int fd = blockIdx.z;
-  const int f = a.nfcore + fd;
-  if (r >= a.nr) return;
-  const int m = a.mval[f];
-  const int am = m < 0 ? -m : m;
-  double2* out = a.y + ((size_t)fd * a.L1 + l) * a.nr + r;
-  if (l < am) {
-    *out = make_double2(0.0, 0.0);
-    return;
-  }
-  const double2* src = mode == 0 ? a.wfn + (size_t)f * a.L1 * a.nr : a.x + (size_t)fd * a.L1 * a.nr;
-  const bool tpart = mode == 0 || mode == 3;
-  const double2* psi_l = src + (size_t)l * a.nr;
-  const int n = a.n;
-  const int jlo = max(0, r - n), jhi = min(a.nr - 1, r + n);
-  const double xr = a.xr[r];
-  const double* al = a.alph + (size_t)(m + a.mmax1) * a.L1;
-  double2 h = make_double2(0.0, 0.0);
-  if (tpart) {
-    const double* band = l == 0 ? a.band_k : a.band_k0;
-    for (int j = jlo; j <= jhi; ++j) {
-      const int d = j - r + n;
-      double2 t;
-      if (d == n) {
-        t = a.tdiag[(size_t)l * a.nr + r];
-      } else {
-        t = make_double2(band[(size_t)d * a.nr + r], 0.0);
-        if (t.x == 0.0) continue;
-      }
-      cfma(h, psi_l[j], t);
-    }
-  }
-  if (mode != 0 || a.isplit == 1) {
-    // the field value: lfield(3) in modes 0 and 3, -c lfield(3) in mode 1
-    const double2 zf = mode == 1 ? cmul(a.zfac1, make_double2(a.lf[2], 0.0)) : make_double2(a.lf[2], 0.0);
-    if (a.igauge == 0) {
-      if (l + 1 < a.L1) cfma(h, psi_l[a.nr + r], cscale(zf, xr * al[l]));
-      if (l - 1 >= am) cfma(h, psi_l[-(ptrdiff_t)a.nr + r], cscale(zf, xr * al[l - 1]));
-    } else {
-      if (l + 1 < a.L1) {
-        const double2* p1 = psi_l + a.nr;
-        double2 dw = make_double2(0.0, 0.0);
-        for (int j = jlo; j <= jhi; ++j) {
-          const double pm = a.band_p[(size_t)(j - r + n) * a.nr + r];
-          if (pm == 0.0) continue;
-          dw.x = fma(p1[j].x, pm, dw.x);
-          dw.y = fma(p1[j].y, pm, dw.y);
-        }
-        cfma(h, dw, cmul(zf, make_double2(0.0, -al[l])));
-        cfma(h, p1[r], cmul(zf, make_double2(0.0, -(al[l] * (l + 1.0)) / xr)));
-      }
-      if (l - 1 >= am) {
-        const double2* p0 = psi_l - a.nr;
-        double2 dw = make_double2(0.0, 0.0);
-        for (int j = jlo; j <= jhi; ++j) {
-          const double pm = a.band_p[(size_t)(j - r + n) * a.nr + r];
-          if (pm == 0.0) continue;
-          dw.x = fma(p0[j].x, pm, dw.x);
-          dw.y = fma(p0[j].y, pm, dw.y);
-        }
-        cfma(h, dw, cmul(zf, make_double2(0.0, -al[l - 1])));
-        cfma(h, p0[r], cscale(cmul(zf, make_double2(0.0, -(al[l - 1] * (double)l) / xr)), -1.0));
-      }
-    }
-  }
-  if (mode == 0) {
-    double2 y = psi_l[r];
-    cfma(y, a.zfac1, h);
-    *out = y;
-  } else if (mode == 3) {
-    *out = cmul(a.zfac1, h);
-  } else {
-    *out = h;
-  }
-}
 
 // Bridge pass, one block per (dynamical orbital, l): the Schur right-hand
 // sides y_B - W_r(k) . y_I(k) - W_l(k+1) . y_I(k+1) (four lanes per bridge),
@@ -333,34 +246,29 @@ int cn_interior_blocks(const CnArgs& a) {
   return a.L1 * nchunk;
 }
 
-void launch_cn_stage(const CnArgs& a, const OneBodyElArgs* ob, int shape, int lc, int mode, hipStream_t s) {
+void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc, int mode, hipStream_t s) {
   const int nd = a.nfun - a.nfcore;
   if (nd <= 0) return;
   if (mode == 3 || mode == 4) {  // y = zfac1 (T + V) x, or zfac1 V x (flag clear)
     if (active_recorder()) return record_unsupported("an application of h1");
-    if (ob) {
-      OneBodyElArgs e = *ob;
-      e.cn = mode == 3 ? 3 : 2;
-      e.cv = a.zfac1;
-      e.stop = a.flag;
-      launch_onebody_el(a.x, a.y, e, s, shape, lc);
-    } else {
-      hipLaunchKernelGGL(k_cn_rhs, dim3((a.nr + 255) / 256, a.L1, nd), dim3(256), 0, s, a, mode == 3 ? 3 : 1);
-    }
+    OneBodyElArgs e = ob;
+    e.cn = mode == 3 ? 3 : 2;
+    e.cv = a.zfac1;
+    e.stop = a.flag;
+    launch_onebody_el(a.x, a.y, e, s, shape, lc);
     return;
   }
-  // with the element right-hand side (stream launches) each term's
-  // convergence test runs at the start of the next term's right-hand side
+  // under stream launches each term's convergence test runs at the start of the next term's right-hand side
   // (the test at the top of h1itr_prop's next cycle) instead of as a launch
   // of its own; a batch records the test as a launch (its series word)
-  const bool fused = ob != nullptr && !active_recorder();
+  const bool fused = !active_recorder();
   if (mode == 2) {  // a plain solve: y = zfac0 psi, then the first term
     if (active_recorder()) return record_unsupported("a rational-function solve");
     launch_zaxpby((size_t)nd * a.L1 * a.nr, a.zfac0, a.wfn + (size_t)a.nfcore * a.L1 * a.nr, make_double2(0.0, 0.0),
                   nullptr, a.y, s);
     mode = 0;
-  } else if (ob) {  // element form of the right-hand side (ndvr = 20)
-    OneBodyElArgs e = *ob;
+  } else {
+    OneBodyElArgs e = ob;
     e.cn = mode + 1;
     if (mode == 1 && fused) {  // the previous term's convergence test first
       e.chk_part = a.part;
@@ -371,9 +279,6 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs* ob, int shape, int lc
       e.chk_flag = a.flag;
     }
     launch_onebody_el(mode == 0 ? a.wfn + (size_t)a.nfcore * a.L1 * a.nr : a.x, a.y, e, s, shape, lc);
-  } else {
-    if (active_recorder()) return record_unsupported("the band right-hand side of the half step (ndvr != 20)");
-    hipLaunchKernelGGL(k_cn_rhs, dim3((a.nr + 255) / 256, a.L1, nd), dim3(256), 0, s, a, mode);
   }
   const int epb = std::min(32, kCnInteriorThreads / a.ni);
   const int nchunk = (a.nfe + epb - 1) / epb;

@@ -350,116 +350,26 @@ __global__ void __launch_bounds__(256) k_legendre(const LegendreJob J) {
 
 // ---------------------------------------------------------------------------
 // One-body part h01 = (T_l + h1) psi (hprod_tprodp, src/hprod/hprod_tprod.F90:152-235;
-// hprod_zprodp, hprod_zprod.F90:108-135; hprod_pzprodp, hprod_pzprod.F90:114-213).
-// Thread per (r, l, orbital).  The FEDVR band is walked with the transposed
-// row bands band[d][r], d = j - r + n.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_onebody(const double2* __restrict__ orb, double2* __restrict__ h01,
-                                                 const OneBodyArgs a) {
-  const double2 zf = make_double2(a.lf[2], 0.0), ef = make_double2(a.lf[5], 0.0);
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const int l = blockIdx.y;
-  const int f = a.f0 + blockIdx.z;
-  if (r >= a.nr || l >= a.L1 || f >= a.f1) return;
-  const int m = a.mval[f];
-  const int am = m < 0 ? -m : m;
-  const bool fc = f < a.nfcore;
-  const int rows = fc ? a.nradfc : a.nr;
-  double2* out = h01 + ((size_t)f * a.L1 + l) * a.nr + r;
-  if (r >= rows || l < am) {
-    *out = make_double2(0.0, 0.0);
-    return;
-  }
-  const int n = a.ndvr;
-  const double2* psi_l = orb + ((size_t)f * a.L1 + l) * a.nr;
-  const double* band = l == 0 ? a.band_k : a.band_k0;
-  const int jlo = max(0, r - n), jhi = min(a.nr - 1, r + n);
-  const double xr = a.xr[r];
-  const double* al = a.alph + (size_t)(m + a.mmax1) * a.L1;
-  double2 h = make_double2(0.0, 0.0);
-  // iprojfc = 1: frozen core gets only the velocity-gauge E.z term
-  // (hprod_htot.F90:100-124)
-  if (fc && !a.fc_full) {
-    if (a.igauge == 1) {
-      if (l + 1 < a.L1) cfma(h, psi_l[a.nr + r], cscale(ef, xr * al[l]));
-      if (l - 1 >= am) cfma(h, psi_l[-(ptrdiff_t)a.nr + r], cscale(ef, xr * al[l - 1]));
-    }
-    *out = h;
-    return;
-  }
-  // kinetic + nuclear + centrifugal (+ frozen-core Hartree) band product
-  for (int j = jlo; j <= jhi; ++j) {
-    int d = j - r + n;
-    double2 t;
-    if (d == n) {
-      t = a.tdiag[(size_t)l * a.nr + r];
-    } else {
-      t = make_double2(band[(size_t)d * a.nr + r], 0.0);
-      if (t.x == 0.0) continue;
-    }
-    cfma(h, psi_l[j], t);
-  }
-  // dipole coupling l +- 1 in the chosen gauge
-  if (a.igauge == 0) {
-    if (l + 1 < a.L1) {
-      double2 tmp = cscale(zf, xr * al[l]);
-      cfma(h, psi_l[a.nr + r], tmp);
-    }
-    if (l - 1 >= am) {
-      double2 tmp = cscale(zf, xr * al[l - 1]);
-      cfma(h, psi_l[-(ptrdiff_t)a.nr + r], tmp);
-    }
-  } else {
-    // d psi at l+1 and l-1 with the radial derivative band
-    if (l + 1 < a.L1) {
-      const double2* p1 = psi_l + a.nr;
-      double2 dw = make_double2(0.0, 0.0);
-      for (int j = jlo; j <= jhi; ++j) {
-        double pm = a.band_p[(size_t)(j - r + n) * a.nr + r];
-        if (pm == 0.0) continue;
-        dw.x = fma(p1[j].x, pm, dw.x);
-        dw.y = fma(p1[j].y, pm, dw.y);
-      }
-      // tmp1 = A * (-i alph), tmp2 = A * (-i alph (l+1) / r)
-      double2 tmp1 = cmul(zf, make_double2(0.0, -al[l]));
-      double2 tmp2 = cmul(zf, make_double2(0.0, -(al[l] * (l + 1.0)) / xr));
-      cfma(h, dw, tmp1);
-      cfma(h, p1[r], tmp2);
-    }
-    if (l - 1 >= am) {
-      const double2* p0 = psi_l - a.nr;
-      double2 dw = make_double2(0.0, 0.0);
-      for (int j = jlo; j <= jhi; ++j) {
-        double pm = a.band_p[(size_t)(j - r + n) * a.nr + r];
-        if (pm == 0.0) continue;
-        dw.x = fma(p0[j].x, pm, dw.x);
-        dw.y = fma(p0[j].y, pm, dw.y);
-      }
-      double2 tmp1 = cmul(zf, make_double2(0.0, -al[l - 1]));
-      double2 tmp2 = cmul(zf, make_double2(0.0, -(al[l - 1] * (double)l) / xr));
-      cfma(h, dw, tmp1);
-      cfma(h, p0[r], cscale(tmp2, -1.0));
-    }
-    // frozen core in the velocity gauge also carries E.z (hprod_htot.F90:123)
-    if (fc) {
-      if (l + 1 < a.L1) cfma(h, psi_l[a.nr + r], cscale(ef, xr * al[l]));
-      if (l - 1 >= am) cfma(h, psi_l[-(ptrdiff_t)a.nr + r], cscale(ef, xr * al[l - 1]));
-    }
-  }
-  *out = h;
-}
-
-// ---------------------------------------------------------------------------
-// One-body part in element-local form (same operator as k_onebody): a block
-// owns GE consecutive elements of one orbital and walks lc consecutive l
-// values.  Lane (element, m) keeps row m of the element's kinetic and d/dr
-// matrices in registers; psi(l-1), psi(l), psi(l+1) of the block's points
-// slide through LDS.  An interior point needs one row product; a bridge adds
-// the last row of the element on its left (the lane after the GE elements
-// recomputes it for the block's first element).  With GE = 3 the block is a
-// single wavefront (63 + 1 lanes) and the bridge partials move by lane
-// shuffles instead of LDS.  The (GE, lc) pair is a launch shape chosen per
-// problem by the autotuner; every shape gives the same bits.  N = ndvr.
+// hprod_zprodp, hprod_zprod.F90:108-135; hprod_pzprodp, hprod_pzprod.F90:114-213)
+// in element-local form: a block of BS threads owns GE = (BS - 1) / (n + 1)
+// consecutive elements of one orbital and walks lc consecutive l values.  Lane
+// (element, m) keeps row m of the element's kinetic and d/dr matrices in
+// registers.  Plane by plane, psi(l) of the block's points goes through LDS
+// and one pass over it gives both T psi(l) and d psi(l)/dr of the lane's row;
+// the output of l takes T(l) and the derivatives of l - 1 and l + 1, which
+// stay in registers.  (The products of psi(l-1) and psi(l+1) used to be formed
+// anew for every l, with three LDS reads per matrix element where one serves
+// now.)  Bound by latency at 3 wavefronts per SIMD: the two matrix rows take
+// 84 registers.  9 orbitals x 64 l x 2399 points, velocity gauge: 98 us beside
+// the mean-field chain of a step and 37 alone, against 134 and 40; the half
+// step's right-hand side in length gauge on 799 points 6.6 against 11.9; n =
+// 17 against the band kernels that n != 20 had: 9 against 26.  An interior point needs one row product; a
+// bridge adds the last row of the element on its left (the lane after the GE
+// elements recomputes it for the block's first element).  A block of 64
+// threads is a single wavefront and its bridge partials move by lane shuffles
+// instead of LDS.  The (BS, lc) pair is a launch shape chosen per problem by
+// the autotuner; every shape gives the same bits.  NM = n for n = 20, else an
+// upper bound of n (16, 24, 32): the rows are padded with zeros.
 // ---------------------------------------------------------------------------
 // The convergence test of a clh1itr term (k_cn_check's arithmetic) in a
 // block of BS threads: the partial sums added by 256 lanes in k_cn_check's
@@ -487,23 +397,25 @@ __device__ __forceinline__ bool cn_series_done(const double* __restrict__ part, 
   return sqrt(tot / nfun) < thresh;
 }
 
-template <int N, int GE, int CN>
+constexpr int onebody_elements(int BS, int n) { return (BS - 1) / (n + 1); }
+
+template <int NM, int BS, int CN>
 __device__ __forceinline__ void onebody_el_body(const double2* __restrict__ orb, double2* __restrict__ h01, const OneBodyElArgs& a, int lc, const Blk bk) {
   if (CN == 2 && a.stop[0]) return;
   if (CN == 2 && a.chk_part) {
-    constexpr int BSC = ((GE * (N + 1) + 1) + 63) / 64 * 64;
-    if (cn_series_done<BSC>(a.chk_part, a.chk_n, a.chk_nfun, a.chk_thresh)) {
+    if (cn_series_done<BS>(a.chk_part, a.chk_n, a.chk_nfun, a.chk_thresh)) {
       if (bk.x == 0 && bk.y == 0 && bk.z == 0 && threadIdx.x == 0) *a.chk_flag = 1;
       return;
     }
   }
   const double2 zf = make_double2(a.lf[2], 0.0), ef = make_double2(a.lf[5], 0.0);
-  constexpr int NP = N + 1;
-  constexpr int BS = ((GE * NP + 1) + 63) / 64 * 64;
   constexpr bool ONE_WAVE = BS == 64;
-  constexpr int TILE = (GE + 1) * N + 1;     // points of elements e0-1 .. e0+GE-1
-  __shared__ double2 sPsi[3][TILE];
-  __shared__ double2 sT[ONE_WAVE ? 1 : BS], sP1[ONE_WAVE ? 1 : BS], sP0[ONE_WAVE ? 1 : BS];
+  constexpr int NPM = NM + 1;
+  constexpr int CAP = BS + 2 * NM;   // points of elements e0-1 .. e0+GE-1, then zeros for padded rows
+  __shared__ double2 sPsi[2][CAP];
+  __shared__ double2 sT[ONE_WAVE ? 1 : BS], sD[ONE_WAVE ? 1 : BS];
+  const int N = NM == 20 ? 20 : a.ndvr, NP = N + 1;
+  const int GE = onebody_elements(BS, N), TILE = (GE + 1) * N + 1;
   const int f = bk.z;
   const int e0 = bk.x * GE;
   const int l0 = bk.y * lc;
@@ -529,173 +441,158 @@ __device__ __forceinline__ void onebody_el_body(const double2* __restrict__ orb,
   const int rows = fc ? a.nradfc : a.nr;
   const int ibase = (e0 - 1) * N - 1;        // global interior index of tile slot 0
   // tile slot of this lane's element point 0
-  const int eslot = (e - (e0 - 1)) * N;
-  double Kr[NP], Pr[NP];
+  const int eslot = lane_ok ? (e - (e0 - 1)) * N : 0;
+  const bool need_t = CN != 2, need_d = a.igauge == 1 && (CN != 1 || a.isplit == 1);
+  const double2* base_f = orb + (size_t)f * a.L1 * a.nr;
+  // l = 0 has its own kinetic matrix of the first element: its difference to
+  // the other l's, applied to psi(0) (ahead of the loop, whose registers the
+  // two matrix rows fill)
+  double2 corr = make_double2(0.0, 0.0);
+  if (need_t && l0 == 0 && lane_ok && e == 0) {
+#pragma unroll 1
+    for (int k = 1; k < NP; ++k) {  // (point 0 is r = 0)
+      const double dk = a.eK0[(size_t)k * NP + m] - a.eK[(size_t)k * NP + m];
+      const double2 x = base_f[k - 1];
+      corr.x = fma(dk, x.x, corr.x);
+      corr.y = fma(dk, x.y, corr.y);
+    }
+  }
+  double Kr[NPM], Pr[NPM];
 #pragma unroll
-  for (int k = 0; k < NP; ++k) {
-    Kr[k] = lane_ok ? a.eK[((size_t)ee * NP + k) * NP + m] : 0.0;
-    Pr[k] = lane_ok ? a.eP[((size_t)ee * NP + k) * NP + m] : 0.0;
+  for (int k = 0; k < NPM; ++k) {
+    const bool ok = lane_ok && k <= N;
+    Kr[k] = ok && need_t ? a.eK[((size_t)ee * NP + k) * NP + m] : 0.0;
+    Pr[k] = ok && need_d ? a.eP[((size_t)ee * NP + k) * NP + m] : 0.0;
   }
   const int i = e * N + m - 1;               // global interior index of (e, m)
   // owner: interior rows, and row 0 of elements >= 1 (the bridge)
   const bool owner = lane_ok && tid < GE * NP && m < N && i >= 0 && i < a.nr;
   const double xr = owner ? a.xr[i] : 1.0;
   const double* al = a.alph + (size_t)(mf + a.mmax1) * a.L1;
-  const double2* base_f = orb + (size_t)f * a.L1 * a.nr;
   // the lane holding the left element's last row: the previous lane, or the
   // extra lane for the first element
   const int pl = tid >= NP ? tid - 1 : GE * NP;
-  auto load_tile = [&](int l, int buf) {
-    for (int q = tid; q < TILE; q += BS) {
-      const int gi = ibase + q;
-      double2 v = make_double2(0.0, 0.0);
-      if (l >= 0 && l < a.L1 && gi >= 0 && gi < a.nr) v = base_f[(size_t)l * a.nr + gi];
-      sPsi[buf][q] = v;
-    }
-  };
-  // plane l + 1 is read from global memory one trip ahead, into registers,
-  // so that its latency overlaps the previous trip's products
-  constexpr int RP = (TILE + BS - 1) / BS;
+  const double2 zero = make_double2(0.0, 0.0);
+  if (NM != 20)  // zeros behind the tile
+    for (int q = TILE + tid; q < CAP; q += BS) sPsi[0][q] = sPsi[1][q] = zero;
+  // plane q is read from global memory one trip ahead, into registers, so
+  // that its latency overlaps the previous plane's products
+  constexpr int RP = 2;
   double2 nx[RP];
-  auto fetch = [&](int l) {
+  auto fetch = [&](int q) {
 #pragma unroll
     for (int j = 0; j < RP; ++j) {
-      const int q = tid + j * BS, gi = ibase + q;
-      nx[j] = (q < TILE && l >= 0 && l < a.L1 && gi >= 0 && gi < a.nr) ? base_f[(size_t)l * a.nr + gi]
-                                                                       : make_double2(0.0, 0.0);
+      const int t = tid + j * BS, gi = ibase + t;
+      nx[j] = (t < TILE && q >= 0 && q < a.L1 && gi >= 0 && gi < a.nr) ? base_f[(size_t)q * a.nr + gi] : make_double2(0.0, 0.0);
     }
   };
-  load_tile(l0, l0 % 3);
-  load_tile(l0 - 1, (l0 + 2) % 3);
-  fetch(l0 + 1);
-  for (int l = l0; l < l1; ++l) {
-    const int b0 = l % 3, b1 = (l + 1) % 3, bm = (l + 2) % 3;
-    __syncthreads();  // the previous trip's reads of buffer b1 are done
+  // own point, T psi and d psi/dr of planes l-1, l and l+1 (completed rows)
+  double2 pd = zero, p0 = zero, pu = zero, Tc = zero, Tn = zero, Dd = zero, Dc = zero, Dn = zero;
+  fetch(l0 - 1);
+#pragma unroll 1
+  for (int q = l0 - 1; q <= l1; ++q) {  // plane q, then the output of l = q - 1
+    double2* buf = sPsi[q & 1];
 #pragma unroll
     for (int j = 0; j < RP; ++j)
-      if (tid + j * BS < TILE) sPsi[b1][tid + j * BS] = nx[j];
-    if (l + 1 < l1) fetch(l + 2);
+      if (tid + j * BS < TILE) buf[tid + j * BS] = nx[j];
+    if (q < l1) fetch(q + 1);
     __syncthreads();
-    // element-row partial products
-    double2 pT = make_double2(0.0, 0.0), pP1 = make_double2(0.0, 0.0), pP0 = make_double2(0.0, 0.0);
-    if (lane_ok && l >= am && CN != 2) {
-      const double2* s0 = sPsi[b0] + eslot;
-      if (l == 0) {
+    pd = p0;
+    p0 = pu;
+    Dd = Dc;
+    Dc = Dn;
+    Tc = Tn;
+    pu = lane_ok ? buf[eslot + m] : make_double2(0.0, 0.0);
+    const bool tq = need_t && q >= l0 && q < l1;
+    double2 pT = zero, pD = zero;
+    const double2* s0 = buf + eslot;
+    if (CN == 2 || !tq) {
+      if (need_d) {
 #pragma unroll
-        for (int k = 0; k < NP; ++k) {
-          const double kk = a.eK0[((size_t)ee * NP + k) * NP + m];
-          pT.x = fma(kk, s0[k].x, pT.x);
-          pT.y = fma(kk, s0[k].y, pT.y);
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < NP; ++k) {
-          pT.x = fma(Kr[k], s0[k].x, pT.x);
-          pT.y = fma(Kr[k], s0[k].y, pT.y);
-        }
-      }
-    }
-    if (lane_ok && l >= am) {
-      if (a.igauge == 1 && (CN != 1 || a.isplit == 1)) {
-        const double2* s1 = sPsi[b1] + eslot;
-        const double2* sm = sPsi[bm] + eslot;
-#pragma unroll
-        for (int k = 0; k < NP; ++k) {
-          pP1.x = fma(Pr[k], s1[k].x, pP1.x);
-          pP1.y = fma(Pr[k], s1[k].y, pP1.y);
-          pP0.x = fma(Pr[k], sm[k].x, pP0.x);
-          pP0.y = fma(Pr[k], sm[k].y, pP0.y);
+        for (int k = 0; k < NPM; ++k) {
+          const double2 x = s0[k];
+          pD.x = fma(Pr[k], x.x, pD.x);
+          pD.y = fma(Pr[k], x.y, pD.y);
         }
       }
+    } else {
+#pragma unroll
+      for (int k = 0; k < NPM; ++k) {
+        const double2 x = s0[k];
+        pT.x = fma(Kr[k], x.x, pT.x);
+        pT.y = fma(Kr[k], x.y, pT.y);
+        pD.x = fma(Pr[k], x.x, pD.x);  // (the rows of d/dr are zero where they are not needed)
+        pD.y = fma(Pr[k], x.y, pD.y);
+      }
+      if (q == 0) pT = cadd(pT, corr);
     }
     // the left neighbour's partials (bridge rows)
-    double2 lT, lP1, lP0;
+    double2 lT, lD;
     if (ONE_WAVE) {
       lT = make_double2(__shfl(pT.x, pl, 64), __shfl(pT.y, pl, 64));
-      lP1 = make_double2(__shfl(pP1.x, pl, 64), __shfl(pP1.y, pl, 64));
-      lP0 = make_double2(__shfl(pP0.x, pl, 64), __shfl(pP0.y, pl, 64));
+      lD = make_double2(__shfl(pD.x, pl, 64), __shfl(pD.y, pl, 64));
     } else {
       sT[tid] = pT;
-      sP1[tid] = pP1;
-      sP0[tid] = pP0;
+      sD[tid] = pD;
       __syncthreads();
       lT = sT[pl];
-      lP1 = sP1[pl];
-      lP0 = sP0[pl];
+      lD = sD[pl];
     }
-    if (owner) {
-      double2 out = make_double2(0.0, 0.0);
-      if (l >= am && i < rows) {
-        double2 T = pT, P1 = pP1, P0 = pP0;
-        if (m == 0) {  // bridge: add the left element's last row
-          T = cadd(T, lT);
-          P1 = cadd(P1, lP1);
-          P0 = cadd(P0, lP0);
-        }
-        const int slot = eslot + m;
-        const double2 p0 = sPsi[b0][slot], pu = sPsi[b1][slot], pd = sPsi[bm][slot];
-        double2 h = make_double2(0.0, 0.0);
-        const bool full = !fc || a.fc_full;
-        if (CN) {
-          // the clh1itr right-hand sides: T psi (CN 1), then V psi (CN 1 with
-          // isplit = 1, and CN 2), as h1itr_prop.F90:57-70,106-114; CN 3
-          // (T + V) psi, hprod_h1tot (hprod_h1tot.F90:2-53)
-          if (CN == 1 || CN == 3) {
-            h = T;
-            cfma(h, p0, a.tzor[(size_t)l * a.nr + i]);
-          }
-          if (CN >= 2 || a.isplit == 1) {
-            if (a.igauge == 0) {
-              if (l + 1 < a.L1) cfma(h, pu, cscale(zf, xr * al[l]));
-              if (l - 1 >= am) cfma(h, pd, cscale(zf, xr * al[l - 1]));
-            } else {
-              if (l + 1 < a.L1) {
-                cfma(h, P1, cmul(zf, make_double2(0.0, -al[l])));
-                cfma(h, pu, cmul(zf, make_double2(0.0, -(al[l] * (l + 1.0)) / xr)));
-              }
-              if (l - 1 >= am) {
-                cfma(h, P0, cmul(zf, make_double2(0.0, -al[l - 1])));
-                cfma(h, pd, cscale(cmul(zf, make_double2(0.0, -(al[l - 1] * (double)l) / xr)), -1.0));
-              }
-            }
-          }
-          double2 y = CN == 1 ? p0 : make_double2(0.0, 0.0);
-          cfma(y, a.cv, h);
-          h01[((size_t)f * a.L1 + l) * a.nr + i] = y;
-          continue;
-        }
-        if (full) {
-          h = T;
-          cfma(h, p0, a.tzor[(size_t)l * a.nr + i]);
-          if (a.igauge == 0) {
-            if (l + 1 < a.L1) cfma(h, pu, cscale(zf, xr * al[l]));
-            if (l - 1 >= am) cfma(h, pd, cscale(zf, xr * al[l - 1]));
-          } else {
-            if (l + 1 < a.L1) {
-              cfma(h, P1, cmul(zf, make_double2(0.0, -al[l])));
-              cfma(h, pu, cmul(zf, make_double2(0.0, -(al[l] * (l + 1.0)) / xr)));
-            }
-            if (l - 1 >= am) {
-              cfma(h, P0, cmul(zf, make_double2(0.0, -al[l - 1])));
-              cfma(h, pd, cscale(cmul(zf, make_double2(0.0, -(al[l - 1] * (double)l) / xr)), -1.0));
-            }
-          }
-        }
-        if (fc && a.igauge == 1) {  // E.z on the frozen core in the velocity gauge
-          if (l + 1 < a.L1) cfma(h, pu, cscale(ef, xr * al[l]));
-          if (l - 1 >= am) cfma(h, pd, cscale(ef, xr * al[l - 1]));
-        }
-        out = h;
+    if (m == 0) {  // bridge: add the left element's last row
+      pT = cadd(pT, lT);
+      pD = cadd(pD, lD);
+    }
+    Tn = pT;
+    Dn = pD;
+    const int l = q - 1;
+    if (l < l0 || !owner) continue;
+    double2 out = zero;
+    if (l >= am && i < rows) {
+      double2 h = zero;
+      // T psi (CN 0, 1, 3; a frozen core with iprojfc = 1 gets only the
+      // velocity-gauge E.z term, hprod_htot.F90:100-124), then the dipole
+      // coupling of l +- 1 in the chosen gauge: CN 1 with isplit = 1 only
+      // (the clh1itr right-hand sides, h1itr_prop.F90:57-70,106-114), CN 2
+      // nothing else, CN 3 (T + V) psi (hprod_h1tot, hprod_h1tot.F90:2-53)
+      const bool full = CN != 0 || !fc || a.fc_full;
+      if (CN != 2 && full) {
+        h = Tc;
+        cfma(h, p0, a.tzor[(size_t)l * a.nr + i]);
       }
-      h01[((size_t)f * a.L1 + l) * a.nr + i] = out;
+      if (CN == 1 ? a.isplit == 1 : full) {
+        if (a.igauge == 0) {
+          if (l + 1 < a.L1) cfma(h, pu, cscale(zf, xr * al[l]));
+          if (l - 1 >= am) cfma(h, pd, cscale(zf, xr * al[l - 1]));
+        } else {
+          if (l + 1 < a.L1) {
+            cfma(h, Dn, cmul(zf, make_double2(0.0, -al[l])));
+            cfma(h, pu, cmul(zf, make_double2(0.0, -(al[l] * (l + 1.0)) / xr)));
+          }
+          if (l - 1 >= am) {
+            cfma(h, Dd, cmul(zf, make_double2(0.0, -al[l - 1])));
+            cfma(h, pd, cscale(cmul(zf, make_double2(0.0, -(al[l - 1] * (double)l) / xr)), -1.0));
+          }
+        }
+      }
+      if (CN == 0 && fc && a.igauge == 1) {  // E.z on the frozen core in the velocity gauge (hprod_htot.F90:123)
+        if (l + 1 < a.L1) cfma(h, pu, cscale(ef, xr * al[l]));
+        if (l - 1 >= am) cfma(h, pd, cscale(ef, xr * al[l - 1]));
+      }
+      if (CN == 0) {
+        out = h;
+      } else {
+        if (CN == 1) out = p0;
+        cfma(out, a.cv, h);
+      }
     }
+    h01[((size_t)f * a.L1 + l) * a.nr + i] = out;
   }
 }
 
-template <int N, int GE, int CN>
-__global__ void __launch_bounds__(((GE * (N + 1) + 1) + 63) / 64 * 64)
+template <int NM, int BS, int CN>
+__global__ void __launch_bounds__(BS, NM <= 20 ? 3 : 2)
     k_onebody_el(const double2* __restrict__ orb, double2* __restrict__ h01, const OneBodyElArgs a, int lc) {
-  onebody_el_body<N, GE, CN>(orb, h01, a, lc, hw_blk());
+  onebody_el_body<NM, BS, CN>(orb, h01, a, lc, hw_blk());
 }
 
 // ---------------------------------------------------------------------------
@@ -1582,51 +1479,44 @@ template void launch_transform_t<float2, double2>(int, const float2*, double2*, 
                                                   const TransformBatch*, int, int, double2*, hipStream_t, int,
                                                   const FcPhaseJob*, int);
 
-// shape: 0 = 3 elements per block (one wavefront), 1 = 6 (128 threads),
-// 2 = 12 (256 threads); lc = l values per block
-template <int CN>
+// shape: 0 = 64 threads (3 elements of 20 rows per block), 1 = 128 (6), 2 =
+// 256 (12); lc = l values per block
+template <int NM, int CN>
 static void launch_onebody_el_t(const double2* orb, double2* h01, const OneBodyElArgs& a, hipStream_t s, int shape,
                                 int lc) {
-  const int nl = (a.L1 + lc - 1) / lc;
+  const int BS = 64 << shape, GE = onebody_elements(BS, a.ndvr);
+  const dim3 grid((a.nfe + GE - 1) / GE, (a.L1 + lc - 1) / lc, a.nfun);
   if (shape == 0)
-    hipLaunchKernelGGL((k_onebody_el<20, 3, CN>), dim3((a.nfe + 2) / 3, nl, a.nfun), dim3(64), 0, s, orb, h01, a, lc);
+    hipLaunchKernelGGL((k_onebody_el<NM, 64, CN>), grid, dim3(64), 0, s, orb, h01, a, lc);
   else if (shape == 1)
-    hipLaunchKernelGGL((k_onebody_el<20, 6, CN>), dim3((a.nfe + 5) / 6, nl, a.nfun), dim3(128), 0, s, orb, h01, a,
-                       lc);
+    hipLaunchKernelGGL((k_onebody_el<NM, 128, CN>), grid, dim3(128), 0, s, orb, h01, a, lc);
   else
-    hipLaunchKernelGGL((k_onebody_el<20, 12, CN>), dim3((a.nfe + 11) / 12, nl, a.nfun), dim3(256), 0, s, orb, h01,
-                       a, lc);
+    hipLaunchKernelGGL((k_onebody_el<NM, 256, CN>), grid, dim3(256), 0, s, orb, h01, a, lc);
 }
 
-bool launch_onebody_el(const double2* orb, double2* h01, const OneBodyElArgs& a, hipStream_t s, int shape, int lc) {
-  if (a.ndvr != 20) return false;
+void launch_onebody_el(const double2* orb, double2* h01, const OneBodyElArgs& a, hipStream_t s, int shape, int lc) {
   lc = std::max(1, std::min(lc, a.L1));
   if (active_recorder()) {
-    const int GE = shape == 0 ? 3 : (shape == 1 ? 6 : 12);
+    if (a.ndvr != 20) return record_unsupported("the one-body part with ndvr != 20");
+    const int BS = 64 << shape, GE = onebody_elements(BS, a.ndvr);
     OneBodyRec r;
     std::memset(&r, 0, sizeof r);
     r.orb = orb; r.h01 = h01; r.a = a; r.lc = lc;
-    const int var[4] = {GE, a.cn, 0, 0};
-    record_launch(kRecOneBody, var, dim3((a.nfe + GE - 1) / GE, (a.L1 + lc - 1) / lc, a.nfun),
-                  ((GE * 21 + 1) + 63) / 64 * 64, 0, r);
-    return true;
+    const int var[4] = {BS, a.cn, 0, 0};
+    record_launch(kRecOneBody, var, dim3((a.nfe + GE - 1) / GE, (a.L1 + lc - 1) / lc, a.nfun), BS, 0, r);
+    return;
   }
-  if (a.cn == 1)
-    launch_onebody_el_t<1>(orb, h01, a, s, shape, lc);
-  else if (a.cn == 2)
-    launch_onebody_el_t<2>(orb, h01, a, s, shape, lc);
-  else if (a.cn == 3)
-    launch_onebody_el_t<3>(orb, h01, a, s, shape, lc);
-  else
-    launch_onebody_el_t<0>(orb, h01, a, s, shape, lc);
-  return true;
-}
-
-void launch_onebody(const double2* orb, double2* h01, const OneBodyArgs& a, hipStream_t s) {
-  if (active_recorder()) return record_unsupported("the band one-body kernel (ndvr != 20)");
-  dim3 block(256);
-  dim3 grid((a.nr + 255) / 256, a.L1, a.f1 - a.f0);
-  hipLaunchKernelGGL(k_onebody, grid, block, 0, s, orb, h01, a);
+  auto by_cn = [&](auto nm) {
+    constexpr int NM = decltype(nm)::value;
+    if (a.cn == 1) launch_onebody_el_t<NM, 1>(orb, h01, a, s, shape, lc);
+    else if (a.cn == 2) launch_onebody_el_t<NM, 2>(orb, h01, a, s, shape, lc);
+    else if (a.cn == 3) launch_onebody_el_t<NM, 3>(orb, h01, a, s, shape, lc);
+    else launch_onebody_el_t<NM, 0>(orb, h01, a, s, shape, lc);
+  };
+  if (a.ndvr == 20) by_cn(std::integral_constant<int, 20>{});
+  else if (a.ndvr <= 16) by_cn(std::integral_constant<int, 16>{});
+  else if (a.ndvr <= 24) by_cn(std::integral_constant<int, 24>{});
+  else by_cn(std::integral_constant<int, 32>{});
 }
 
 // Bridge pass of the Poisson solve, one block per (pair, L), for grids
@@ -2680,15 +2570,15 @@ __global__ void __launch_bounds__(256) k_legendre_batch(const LegendreJob* __res
   });
 }
 
-template <int GE, int CN>
-__global__ void __launch_bounds__(((GE * 21 + 1) + 63) / 64 * 64)
+template <int BS, int CN>
+__global__ void __launch_bounds__(BS, CN == 2 ? 3 : 2)
     k_onebody_el_batch(const OneBodyRec* __restrict__ recs, const BatchMap map) {
   __shared__ __align__(16) unsigned char raw[sizeof(OneBodyRec)];
   int have = -1;
   batch_walk(map, [&](int m) { return CN == 2 && (gate_closed(recs[m].gate) || recs[m].a.stop[0] != 0); },
              [&](int m, const Blk& bk) {
     const OneBodyRec& r = stage_rec(recs, m, raw, have);
-    onebody_el_body<20, GE, CN>(r.orb, r.h01, r.a, r.lc, bk);
+    onebody_el_body<20, BS, CN>(r.orb, r.h01, r.a, r.lc, bk);
   });
 }
 
@@ -2914,15 +2804,15 @@ bool launch_batch_kernels(const LaunchRec& p, const void* recs, const BatchMap& 
     }
     case kRecOneBody: {
       switch (p.var[0] * 10 + p.var[1]) {
-        case 30: TD1C_BATCH((k_onebody_el_batch<3, 0>), OneBodyRec); return true;
-        case 31: TD1C_BATCH((k_onebody_el_batch<3, 1>), OneBodyRec); return true;
-        case 32: TD1C_BATCH((k_onebody_el_batch<3, 2>), OneBodyRec); return true;
-        case 60: TD1C_BATCH((k_onebody_el_batch<6, 0>), OneBodyRec); return true;
-        case 61: TD1C_BATCH((k_onebody_el_batch<6, 1>), OneBodyRec); return true;
-        case 62: TD1C_BATCH((k_onebody_el_batch<6, 2>), OneBodyRec); return true;
-        case 120: TD1C_BATCH((k_onebody_el_batch<12, 0>), OneBodyRec); return true;
-        case 121: TD1C_BATCH((k_onebody_el_batch<12, 1>), OneBodyRec); return true;
-        case 122: TD1C_BATCH((k_onebody_el_batch<12, 2>), OneBodyRec); return true;
+        case 640: TD1C_BATCH((k_onebody_el_batch<64, 0>), OneBodyRec); return true;
+        case 641: TD1C_BATCH((k_onebody_el_batch<64, 1>), OneBodyRec); return true;
+        case 642: TD1C_BATCH((k_onebody_el_batch<64, 2>), OneBodyRec); return true;
+        case 1280: TD1C_BATCH((k_onebody_el_batch<128, 0>), OneBodyRec); return true;
+        case 1281: TD1C_BATCH((k_onebody_el_batch<128, 1>), OneBodyRec); return true;
+        case 1282: TD1C_BATCH((k_onebody_el_batch<128, 2>), OneBodyRec); return true;
+        case 2560: TD1C_BATCH((k_onebody_el_batch<256, 0>), OneBodyRec); return true;
+        case 2561: TD1C_BATCH((k_onebody_el_batch<256, 1>), OneBodyRec); return true;
+        case 2562: TD1C_BATCH((k_onebody_el_batch<256, 2>), OneBodyRec); return true;
         default: return false;
       }
     }

@@ -40,18 +40,6 @@ struct TransformBatch {
   int odd;         // |m| & 1
 };
 
-struct OneBodyArgs {
-  int nr, L1, ndvr, nfcore, nradfc, f0, f1, mmax1, igauge, fc_full;
-  const int* mval;
-  const double* band_k;   // [2n+1][nr] kinetic band for l = 0
-  const double* band_k0;  // [2n+1][nr] kinetic band for l >= 1
-  const double* band_p;   // [2n+1][nr] d/dr band
-  const double* xr;       // [nr]
-  const double* alph;     // [2mmax1+1][L1]
-  const double2* tdiag;   // [L1][nr]
-  const double* lf;       // device lfield[9]: [2] gauge field, [5] E (frozen-core length term)
-};
-
 struct OneBodyElArgs {
   int nr, nfe, L1, ndvr, nfcore, nradfc, nfun, mmax1, igauge, fc_full;
   const int* mval;
@@ -86,9 +74,6 @@ struct OneBodyElArgs {
 struct CnArgs {
   int nr, n, nfe, ni, nb, K, L1, nfun, nfcore, mmax1, igauge, isplit;
   const int* mval;
-  const double *band_k, *band_k0, *band_p;  // [2n+1][nr] transposed bands
-  const double2* tdiag;                     // [L1][nr] tmat diagonal (+ v2jfc)
-  const double *xr, *alph;
   const double* lf;                         // device lfield[9] of this half step
   const double2 *G;                         // [L1][gstride][k][i] = G_e(i, k)
   int gstride;                              // elements per l in G (nfe, or more in a shared table)
@@ -114,9 +99,9 @@ int cn_interior_blocks(const CnArgs& a);
 // of a plain solve, right-hand side zfac0 psi; mode 3: only the right-hand
 // side y = zfac1 (T + V) x, an application of h1 (x, y of the arguments);
 // mode 4: only y = zfac1 V x (flag[0] must be clear)
-// ob: the element one-body arguments for the right-hand side (ndvr = 20),
-// with its launch shape; null for the band kernel
-void launch_cn_stage(const CnArgs& a, const OneBodyElArgs* ob, int shape, int lc, int mode, hipStream_t s);
+// ob: the element one-body arguments for the right-hand side, with its launch
+// shape
+void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc, int mode, hipStream_t s);
 // the convergence test of the term just enqueued (mode 1: kept set once set)
 void launch_cn_check(const CnArgs& a, hipStream_t s);
 
@@ -279,10 +264,10 @@ template <class TI, class TO>
 void launch_transform_t(int mode, const TI* in, TO* out, const LegendreMats& M, const TransformBatch* batch, int nbatch,
                         int nr, double2* copy, hipStream_t s, int path = 0, const FcPhaseJob* fc = nullptr,
                         int tvar = 1);
-void launch_onebody(const double2* orb, double2* h01, const OneBodyArgs& a, hipStream_t s);
-// shape 0/1/2: 3/6/12 elements per block; lc: l values per block (any
-// shape gives the same bits; the autotuner picks one per problem)
-bool launch_onebody_el(const double2* orb, double2* h01, const OneBodyElArgs& a, hipStream_t s, int shape = 2,
+// shape 0/1/2: 64/128/256 threads per block (3/6/12 elements of 20 rows); lc:
+// l values per block (any shape gives the same bits; the autotuner picks one
+// per problem)
+void launch_onebody_el(const double2* orb, double2* h01, const OneBodyElArgs& a, hipStream_t s, int shape = 2,
                        int lc = 2);
 template <class T>  // rho and v complex128 or complex64; the solve is FP64
 void launch_poisson(const T* rho, double2* xb, T* v, const PoissonArgs& a, hipStream_t s, int part = 0);  // part 1 bridge pass, 2 interior pass, 0 both
@@ -469,7 +454,7 @@ __device__ __forceinline__ const R& stage_rec(const R* __restrict__ recs, int m,
 
 enum RecKind {
   kRecLegendre = 1,     // var: direction (1 theta -> l) + 2 (pair products), row tiles, type code
-  kRecOneBody,          // var: GE, CN
+  kRecOneBody,          // var: threads, CN
   kRecPoissonBridge,    // var: type code (LDS form, ndvr = 20)
   kRecPoissonInterior,  // var: type code
   kRecMfprodT,          // var: NF, type code (dynamical cores only)

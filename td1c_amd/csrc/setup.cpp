@@ -379,13 +379,11 @@ bool Setup::build(const td1c_problem& p) {
   // ---- kernel-side one-body tables ----
   xr.assign(nr, 0);
   for (int i = 0; i < nr; ++i) xr[i] = xrad[i + 1];
-  bandT_k.assign(bw * nr, 0); bandT_k0.assign(bw * nr, 0); bandT_p.assign(bw * nr, 0);
+  bandT_p.assign(bw * nr, 0);
   for (int i = 0; i < nr; ++i)
     for (int d = 0; d < (int)bw; ++d) {
       int j = i + d - n;
       if (j < 0 || j >= nr) continue;
-      bandT_k[(size_t)d * nr + i] = radk[bw * (i + 1) + d];
-      bandT_k0[(size_t)d * nr + i] = radk0[bw * (i + 1) + d];
       bandT_p[(size_t)d * nr + i] = radp[bw * (i + 1) + d];
     }
   // diagonal of tmat (bas_gen_tmat, src/bas/bas_gen_tmat.F90:63-118): the

@@ -36,9 +36,7 @@ struct Setup {
 
   // kernel tables ---------------------------------------------------------
   std::vector<double> xr;        // interior r, nr
-  std::vector<double> bandT_k;   // [2n+1][nr]: radk row band, transposed (l = 0)
-  std::vector<double> bandT_k0;  // [2n+1][nr]: radk0 row band (l >= 1)
-  std::vector<double> bandT_p;   // [2n+1][nr]: radp row band
+  std::vector<double> bandT_p;   // [2n+1][nr]: radp row band, transposed
   std::vector<double> tdiag;     // [L1][nr] complex (re,im): diagonal of tmat
   std::vector<double> tzor;      // [L1][nr] complex (re,im): tmat diagonal without the kinetic part
   // element-local matrices [u][k][m] (m fastest) of the distinct elements

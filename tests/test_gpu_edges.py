@@ -55,3 +55,28 @@ def test_partitions(gpu_lib, nfc, ndc, nact, nel, precision):
     prob = Problem(nfe=3, ndvr=20, rmax=9.0, lmax1=3, lmax2=6, znuc=4.0, nfcore1=nfc, ndcore=ndc, nact=nact, nel_alpha=n,
                    nel_beta=n, lval=[0] * (nfc + ndc + nact), igauge=1, precision=precision)
     assert hprod_error(prob, C.LF_VEL) < (1e-5 if precision else 1e-11)
+
+
+# the element one-body kernel at orders other than 20 (rows padded to 16, 24
+# and 32) and element counts that end inside a block, both gauges, a frozen
+# core beside m = 0 and 1; the half step's right-hand sides with it
+@pytest.mark.parametrize("igauge", [0, 1])
+@pytest.mark.parametrize("ndvr,nfe", [(2, 5), (5, 24), (15, 4), (16, 13), (17, 3), (20, 13), (24, 7), (25, 2), (32, 8)])
+def test_onebody_orders(gpu_lib, ndvr, nfe, igauge):
+    import torch
+
+    prob = Problem(nfe=nfe, ndvr=ndvr, rmax=1.5 * nfe, lmax1=3, lmax2=6, znuc=5.0, nfcore1=1, ndcore=2, nel_alpha=3,
+                   nel_beta=3, mval=[0, 0, 1], lval=[0, 0, 1], igauge=igauge, isplit=1)
+    lf = C.LF_VEL if igauge else C.LF_LEN
+    assert hprod_error(prob, lf) < 1e-11
+    o = Oracle(prob)
+    w = C.smooth_wfn_for(prob, o.lcic)
+    o.set_wfn0(w)
+    o.h1itr_gen(0.005)
+    ref, _ = o.h1itr_prop(lf, 0.005, w)
+    hp = td1c_amd.HProd(prob)
+    hp.set_wfn0(w)
+    hp.h1itr_gen(0.01)
+    got = hp.h1itr_prop(lf, hp.to_device(w))
+    torch.cuda.synchronize()
+    assert np.linalg.norm(got.cpu().numpy() - ref) < 1e-11 * np.linalg.norm(ref)
