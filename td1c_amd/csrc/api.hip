@@ -130,7 +130,11 @@ struct td1c_ctx {
   // cn_dt / 2, the series terms and the convergence flag
   double cn_dt = 0.0;
   int cn_maxcyc = 20;
-  int* cn_flag_host = nullptr;  // pinned: the series' flag read back by stream launches
+  // terms that the last series of each slot took (pinned, written by the
+  // device), the terms to launch, and how often fewer would have done
+  static constexpr int kSeries = 24;
+  int* cn_count_host = nullptr;
+  int cn_want[kSeries] = {}, cn_low[kSeries] = {}, cn_since = 0;
   double cn_thresh = 1.0e-10;
   int cn_K = 0, cn_npart1 = 0;
   DevBuf<double2> cnG, cnWl, cnWr, cnPa, cnPg, cnBinv, cn_x, cn_y;
@@ -249,7 +253,7 @@ struct td1c_ctx {
     DevBuf<float>* fm[] = {&m_g2L_f, &m_L2g_f, &k_g2L_f, &k_L2g_f};
     for (auto* b : fm) b->release();
     if (gexec) (void)hipGraphExecDestroy(gexec);
-    if (cn_flag_host) (void)hipHostFree(cn_flag_host);
+    if (cn_count_host) (void)hipHostFree(cn_count_host);
     if (cap_stream) (void)hipStreamDestroy(cap_stream);
     for (auto& e : fj)
       if (e) (void)hipEventDestroy(e);
@@ -2024,6 +2028,7 @@ static int cn_prepare(td1c_ctx* c, double dtime) {
     HIP_TRY(c->cn_part.alloc(npart));
   }
   c->cn_dt = dtime;
+  c->cn_want[0] = 0;
   return 0;
 }
 
@@ -2047,27 +2052,54 @@ static CnArgs cn_args(td1c_ctx* c, const double* d_lf, double2* wfn) {
 
 // maxcyc more terms (mode 1) of a series whose first term is enqueued.
 // A captured or recorded step holds every term (the converged ones return
-// at once).  Under stream launches, after the second term and every two
-// terms after that, the host reads the flag back (the call waits for the
-// device to get there) and stops enqueuing once the series has converged:
-// the later terms would all return at once, and each would still cost its
-// launches.
-static int enqueue_series(td1c_ctx* c, const CnArgs& a, const OneBodyElArgs& obp, int maxcyc, hipStream_t s) {
+// at once).  Under stream launches the call enqueues one term more than the
+// longest of the slot's recent series took, as far as their counts have
+// arrived, and k_cn_tail, which forms whatever is still missing: any choice
+// gives the same bits, and no call waits for the device.  A converged term
+// costs its three launches (about 9 us), a missing one is formed slowly, so
+// the choice follows an increase at once and a decrease after 64 series, and
+// the host waits for the device once in 16 series, so that the counts it has
+// are of a step or two before.  The first series of a slot (of new factors)
+// reads the count back after the second term and every two terms after.
+static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& obp, int maxcyc, int slot, hipStream_t s) {
+  CnArgs a = a0;
+  auto term = [&](int k) {
+    a.term = k;
+    launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 1, s);
+  };
   if (c->capturing || active_recorder()) {
-    for (int k = 0; k < maxcyc; ++k) launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 1, s);
+    for (int k = 1; k <= maxcyc; ++k) term(k);
     return 0;
   }
-  if (!c->cn_flag_host) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_flag_host), sizeof(int)));
-  int k = 0;
-  while (k < maxcyc) {
-    const int chunk = k == 0 ? 1 : 2;
-    for (int j = 0; j < chunk && k < maxcyc; ++j, ++k) launch_cn_stage(a, obp, c->ob_shape, c->ob_lc, 1, s);
-    if (k >= maxcyc) break;
-    launch_cn_check(a, s);
-    HIP_TRY(hipMemcpyAsync(c->cn_flag_host, a.flag, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (*c->cn_flag_host) break;
+  if (slot < 0 || slot >= td1c_ctx::kSeries) slot = 0;
+  if (!c->cn_count_host)
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), td1c_ctx::kSeries * sizeof(int)));
+  volatile int* count = c->cn_count_host + slot;
+  if (c->cn_want[slot] == 0) {
+    *count = 0;
+    for (int k = 0; k < maxcyc;) {
+      const int chunk = k == 0 ? 1 : 2;
+      for (int j = 0; j < chunk && k < maxcyc; ++j) term(++k);
+      launch_cn_tail(a, obp, c->ob_lc, k, k, c->cn_count_host + slot, s);  // the test alone
+      HIP_TRY(hipStreamSynchronize(s));
+      if (*count >= 0) break;
+    }
+    const int n = *count;
+    c->cn_want[slot] = (n >= 0 ? n : -1 - n) + 1;
+    return 0;
   }
+  if (++c->cn_since >= 16) {
+    HIP_TRY(hipStreamSynchronize(s));
+    c->cn_since = 0;
+  }
+  const int n = *count, need = (n >= 0 ? n : -1 - n) + 1;
+  if (need >= c->cn_want[slot] || ++c->cn_low[slot] >= 64) {
+    c->cn_want[slot] = need;
+    c->cn_low[slot] = 0;
+  }
+  const int m = std::min(maxcyc, c->cn_want[slot]);
+  for (int k = 1; k <= m; ++k) term(k);
+  launch_cn_tail(a, obp, c->ob_lc, m, maxcyc, c->cn_count_host + slot, s);
   return 0;
 }
 
@@ -2087,7 +2119,7 @@ static int enqueue_h1itr(td1c_ctx* c, const double* d_lf, double2* wfn, hipStrea
   ob.stop = a.flag;
   TIMED("h1itr");
   launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, 0, s);
-  return enqueue_series(c, a, ob, c->cn_maxcyc, s);
+  return enqueue_series(c, a, ob, c->cn_maxcyc, 0, s);
 }
 
 static int enqueue_rk_step(td1c_ctx* c, int rk_order, double dtime, const double* d_lf, double2* wfn, int apply_mask,
@@ -2597,6 +2629,7 @@ int etd_generate(td1c_ctx* c, int scheme, double dt, int rosen, int maxcyc, doub
   }
   c->etd_tabs.clear();
   c->etd_ready = false;
+  for (int& w : c->cn_want) w = 0;
   if (scheme == 1) {
     const int fam[kEtdRats] = {0, 0, 1, 1, 2, 2, 3};
     const double dts[kEtdRats] = {dt, 0.5 * dt, dt, 0.5 * dt, dt, 0.5 * dt, dt};
@@ -2720,7 +2753,7 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
     }
   };
   // the denominator factors of R on the dynamical rows of orb, in place
-  int series_err = 0;  // a failed read-back of a series flag (enqueue_series)
+  int series_err = 0;  // a failed allocation of enqueue_series
   auto denom = [&](const td1c_ctx::EtdRat& R) {
     for (int i = 0; i < R.dimd; ++i) {
       if (R.tab[i] < 0) continue;
@@ -2737,7 +2770,7 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
       ob.stop = a.flag;
       launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, 2, s);
       if (S.isplit == 1 && S.icomp == 1)
-        if (int rc = enqueue_series(c, a, ob, c->etd_maxcyc, s)) series_err = rc;
+        if (int rc = enqueue_series(c, a, ob, c->etd_maxcyc, 1 + 3 * (int)(&R - c->etd) + i, s)) series_err = rc;
     }
   };
   auto cmulh = [](double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
@@ -2843,7 +2876,7 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
       ob.cv = a.zfac1;
       ob.stop = a.flag;
       launch_cn_stage(a, ob, c->ob_shape, c->ob_lc, 2, s);
-      if (int rc = enqueue_series(c, a, ob, c->etd_maxcyc, s)) series_err = rc;
+      if (int rc = enqueue_series(c, a, ob, c->etd_maxcyc, 0, s)) series_err = rc;
       launch_zaxpby(so, make_double2(-1.0, 0.0), in, make_double2(2.0, 0.0), out, out, s);
     };
     const double dt = c->etd_dt;

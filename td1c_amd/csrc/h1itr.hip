@@ -22,6 +22,7 @@
 
 #include "devmath.hpp"
 #include "kernels.hpp"
+#include "onebody.hpp"
 
 namespace td1c {
 
@@ -201,6 +202,7 @@ __device__ __forceinline__ void cn_interior_body(const CnArgs& a, int mode, int 
 #pragma unroll
     for (int w = 0; w < BS / 64; ++w) s += sRed[w];
     a.part[a.npart1 + bk.x] = s;
+    if (bk.x == 0) a.flag[1] = a.term;
   }
 }
 
@@ -231,10 +233,6 @@ __device__ __forceinline__ void cn_check_body(const CnArgs& a, int mode, int nbl
   }
 }
 
-__global__ void __launch_bounds__(kCnInteriorThreads) k_cn_check(const CnArgs a, int mode, int nblk) {
-  cn_check_body(a, mode, nblk);
-}
-
 template <int NI>
 __global__ void __launch_bounds__(kCnInteriorThreads) k_cn_interior(const CnArgs a, int mode, int epb, int nchunk) {
   cn_interior_body<NI>(a, mode, epb, nchunk, hw_blk());
@@ -244,6 +242,15 @@ int cn_interior_blocks(const CnArgs& a) {
   const int epb = std::min(32, kCnInteriorThreads / a.ni);
   const int nchunk = (a.nfe + epb - 1) / epb;
   return a.L1 * nchunk;
+}
+
+// the convergence test of the term in a.part, for a right-hand side to make
+static void cn_check_args(const CnArgs& a, OneBodyElArgs& e) {
+  e.chk_part = a.part;
+  e.chk_n = a.npart1 + cn_interior_blocks(a);
+  e.chk_nfun = a.nfun;
+  e.chk_thresh = a.thresh;
+  e.chk_flag = a.flag;
 }
 
 void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc, int mode, hipStream_t s) {
@@ -271,12 +278,7 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc
     OneBodyElArgs e = ob;
     e.cn = mode + 1;
     if (mode == 1 && fused) {  // the previous term's convergence test first
-      e.chk_part = a.part;
-      e.chk_n = a.npart1 + a.L1 * ((a.nfe + std::min(32, kCnInteriorThreads / a.ni) - 1) /
-                                   std::min(32, kCnInteriorThreads / a.ni));
-      e.chk_nfun = a.nfun;
-      e.chk_thresh = a.thresh;
-      e.chk_flag = a.flag;
+      cn_check_args(a, e);
     }
     launch_onebody_el(mode == 0 ? a.wfn + (size_t)a.nfcore * a.L1 * a.nr : a.x, a.y, e, s, shape, lc);
   }
@@ -299,13 +301,74 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc
     hipLaunchKernelGGL((k_cn_interior<19>), grid, dim3(kCnInteriorThreads), 0, s, a, mode, epb, nchunk);
   else
     hipLaunchKernelGGL((k_cn_interior<0>), grid, dim3(kCnInteriorThreads), 0, s, a, mode, epb, nchunk);
-  if (!fused) hipLaunchKernelGGL(k_cn_check, dim3(1), dim3(kCnInteriorThreads), 0, s, a, mode, (int)grid.x);
 }
 
-void launch_cn_check(const CnArgs& a, hipStream_t s) {
-  const int epb = std::min(32, kCnInteriorThreads / a.ni);
-  const int nblk = a.L1 * ((a.nfe + epb - 1) / epb);
-  hipLaunchKernelGGL(k_cn_check, dim3(1), dim3(kCnInteriorThreads), 0, s, a, 1, nblk);
+// The end of a series under stream launches, one block: the convergence test
+// of the last term launched, and while it fails the further terms, the blocks
+// of their three launches walked one after the other (the same bits; slow, and
+// reached only when a series grows by more than the terms the host added to
+// what the previous ones took).  The number of terms (-1 - it when the series
+// has not converged) goes to pinned host memory for the next call's choice, so
+// that no call waits for the device: the test as a launch, the copy of its flag
+// and the wait took about 35 us per half step (8 steps of a He problem on 799
+// points 4.56 -> 3.97 ms).
+template <int NM>
+__global__ void __launch_bounds__(256) k_cn_tail(const CnArgs a, const OneBodyElArgs e, int lc, int term0, int maxcyc,
+                                                 int epb, int nchunk, int* __restrict__ count) {
+  const int nd = a.nfun - a.nfcore;
+  int last = a.flag[1];
+  bool done = a.flag[0] != 0;
+  if (!done) {
+    OneBodyElArgs r = e;
+    r.chk_part = nullptr;  // (tested here)
+    const int GE = onebody_elements(256, a.n);
+    const int nx = (a.nfe + GE - 1) / GE, ny = (a.L1 + lc - 1) / lc;
+    for (int term = term0 + 1;; ++term) {
+      __syncthreads();
+      if (cn_series_done<256>(e.chk_part, e.chk_n, e.chk_nfun, e.chk_thresh)) {
+        if (threadIdx.x == 0) a.flag[0] = 1;
+        done = true;
+        break;
+      }
+      if (term > maxcyc) break;
+#pragma unroll 1
+      for (int b = 0; b < nx * ny * nd; ++b) {
+        __syncthreads();
+        onebody_el_body<NM, 256, 2>(a.x, a.y, r, lc, Blk{b % nx, (b / nx) % ny, b / (nx * ny), nx, ny, nd});
+      }
+      __threadfence_block();
+#pragma unroll 1
+      for (int b = 0; b < nd * a.L1; ++b) {
+        __syncthreads();
+        cn_bridge_body<256>(a, 1, Blk{b, 0, 0, nd * a.L1, 1, 1});
+      }
+      __threadfence_block();
+#pragma unroll 1
+      for (int b = 0; b < a.L1 * nchunk; ++b) {
+        __syncthreads();
+        cn_interior_body<NM == 20 ? 19 : 0>(a, 1, epb, nchunk, Blk{b, 0, 0, a.L1 * nchunk, 1, 1});
+      }
+      __threadfence_block();
+      last = term;
+    }
+  }
+  if (threadIdx.x == 0) *count = done ? last : -1 - last;
+}
+
+void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
+                    hipStream_t s) {
+  const int epb = std::min(32, kCnInteriorThreads / a.ni), nchunk = (a.nfe + epb - 1) / epb;
+  OneBodyElArgs e = ob;
+  e.cn = 2;
+  cn_check_args(a, e);
+  lc = std::max(1, std::min(lc, a.L1));
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, dim3(1), dim3(256), 0, s, a, e, lc, term0, maxcyc, epb, nchunk, count);
+  };
+  if (a.n == 20) go(k_cn_tail<20>);
+  else if (a.n <= 16) go(k_cn_tail<16>);
+  else if (a.n <= 24) go(k_cn_tail<24>);
+  else go(k_cn_tail<32>);
 }
 
 __global__ void __launch_bounds__(256) k_cn_bridge_batch(const CnRec* __restrict__ recs, const BatchMap map) {

@@ -86,7 +86,8 @@ struct CnArgs {
   double2 zfac1;                            // -c
   double2 zfac0;                            // mode 2: the first right-hand side zfac0 psi
   double thresh;
-  int* flag;                                // [0] converged
+  int* flag;                                // [0] converged, [1] the last term formed
+  int term;                                 // the term a launch forms (0: the first)
   double* part;                             // norm partial sums: bridge jobs, then interior blocks
   int npart1;
 };
@@ -102,8 +103,11 @@ int cn_interior_blocks(const CnArgs& a);
 // ob: the element one-body arguments for the right-hand side, with its launch
 // shape
 void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc, int mode, hipStream_t s);
-// the convergence test of the term just enqueued (mode 1: kept set once set)
-void launch_cn_check(const CnArgs& a, hipStream_t s);
+// after term0 later terms: the convergence test of the last one and the terms
+// still missing up to maxcyc; the number n formed goes to *count (host
+// memory), -1 - n when the series has not converged
+void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
+                    hipStream_t s);
 
 struct PoissonArgs {
   int nr, n, nfe, ni, L2, npair;
