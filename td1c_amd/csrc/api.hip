@@ -775,9 +775,15 @@ struct CiStage {
 void enqueue_orbin_theta(td1c_ctx* c, const double* d_lf, const double2* wfn, hipStream_t s);
 void enqueue_orbin_fc_l(td1c_ctx* c, hipStream_t sfc);
 
-void enqueue_orbin(td1c_ctx* c, const double* d_lf, const double2* wfn, hipStream_t s) {
+// Returns the l-space orbitals for the observables: without frozen cores the
+// state itself, read in place (the launch that copied it also formed the theta
+// grid, which they do not use: the three dipole forms and the ionisation
+// probabilities of 9 orbitals on 2399 points, l up to 63: 377 -> 326 us).
+const double2* enqueue_orbin(td1c_ctx* c, const double* d_lf, const double2* wfn, hipStream_t s) {
+  if (c->S.nfcore == 0) return wfn;
   enqueue_orbin_theta(c, d_lf, wfn, s);
   enqueue_orbin_fc_l(c, s);
+  return c->orb;
 }
 
 void enqueue_orbin_theta(td1c_ctx* c, const double* d_lf, const double2* wfn, hipStream_t s) {
@@ -1543,13 +1549,13 @@ static int enqueue_dipole(td1c_ctx* c, int nforms, const double* lfield, const d
   hipStream_t s = (hipStream_t)stream;
   Setup& S = c->S;
   HIP_TRY(hipMemcpyAsync(c->lf_dev.p, lfield, 9 * sizeof(double), hipMemcpyHostToDevice, s));
-  enqueue_orbin(c, c->lf_dev.p, reinterpret_cast<const double2*>(d_wfn), s);
+  const double2* orb = enqueue_orbin(c, c->lf_dev.p, reinterpret_cast<const double2*>(d_wfn), s);
   IslandArgs ia = island_args(c, reinterpret_cast<const double2*>(d_cic), 1.0);
   if (S.nact > 0) launch_island_a(ia, s);
   DipoleArgs a{};
   a.nr = S.nr; a.L1 = S.L1; a.nfun = S.nfun; a.nfcore = S.nfcore; a.ncore = S.ncore; a.nact = S.nact;
   a.nradfc = S.nradfc; a.mmax1 = S.mmax1; a.mval = c->mval.p; a.xr = c->xr.p; a.alph = c->alph.p;
-  a.orb = c->orb; a.den1 = c->den1.p;
+  a.orb = orb; a.den1 = c->den1.p;
   a.ndvr = S.n; a.igauge = S.igauge; a.znuc = S.znuc; a.nel = (double)S.nel[2];
   a.band_p = c->band_p.p; a.lf = c->lf_dev.p;
   launch_dipole(a, nforms, c->dip_part.p, d_out, s);
@@ -1697,7 +1703,7 @@ static int ipx_distribution(td1c_ctx* c, double rad, const double* lfield, const
   if (S.nfcore > 0 && !c->wfn0_set) return fail(-4, "frozen core needs td1c_set_wfn0 first");
   if (S.nact > 0 && !d_cic) return fail(-1, "null CI vector");
   HIP_TRY(hipMemcpyAsync(c->lf_dev.p, lfield, 9 * sizeof(double), hipMemcpyHostToDevice, s));
-  enqueue_orbin(c, c->lf_dev.p, reinterpret_cast<const double2*>(d_wfn), s);
+  const double2* orb = enqueue_orbin(c, c->lf_dev.p, reinterpret_cast<const double2*>(d_wfn), s);
   int cut = S.nr;
   for (int i = 0; i < S.nr; ++i)
     if (S.xr[i] > rad) {
@@ -1705,7 +1711,7 @@ static int ipx_distribution(td1c_ctx* c, double rad, const double* lfield, const
       break;
     }
   const int nf = S.nfun;
-  launch_window_ovlp(c->orb, c->mval.p, nf, S.nr, S.L1, cut, c->ovlp.p, s);
+  launch_window_ovlp(orb, c->mval.p, nf, S.nr, S.L1, cut, c->ovlp.p, s);
   HIP_TRY(hipGetLastError());
   std::vector<std::complex<double>> ov((size_t)nf * nf), cic(S.nact > 0 ? S.lcic : 1, 1.0);
   HIP_TRY(hipMemcpyAsync(ov.data(), c->ovlp.p, ov.size() * sizeof(double2), hipMemcpyDeviceToHost, s));

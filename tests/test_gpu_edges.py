@@ -80,3 +80,24 @@ def test_onebody_orders(gpu_lib, ndvr, nfe, igauge):
     got = hp.h1itr_prop(lf, hp.to_device(w))
     torch.cuda.synchronize()
     assert np.linalg.norm(got.cpu().numpy() - ref) < 1e-11 * np.linalg.norm(ref)
+
+
+# the observables without frozen cores read the state in place: after an hprod
+# of another state, and with rows below l = |m| that no orbital has
+@pytest.mark.parametrize("igauge,nact", [(0, 0), (1, 0), (1, 2)])
+def test_observables_in_place(gpu_lib, igauge, nact):
+    prob = Problem(nfe=5, ndvr=20, rmax=15.0, lmax1=4, lmax2=8, znuc=4.0, ndcore=2 - nact // 2, nact=nact, nel_alpha=2,
+                   nel_beta=2, mval=[0, 1] if nact == 0 else [0, 0, 1], igauge=igauge)
+    lf = C.LF_VEL if igauge else C.LF_LEN
+    o = Oracle(prob)
+    w = C.wfn_for(prob, o.lcic)
+    rows = w[:prob.nfun * 5 * prob.nr].reshape(prob.nfun, 5, prob.nr)
+    ref, ref_p = o.dipole3(lf, w), o.ipx(2, 4.0, lf, w)
+    rows[-1, 0] = 7.0
+    hp = td1c_amd.HProd(prob)
+    d = hp.to_device(w)
+    hp.htot(1.0, lf, hp.to_device(w * 0.5))
+    scale = max(1.0, np.abs(ref).max())
+    assert np.abs(hp.dipole3(lf, d) - ref).max() <= 1e-11 * scale
+    assert np.abs(hp.ipx(2, 4.0, lf, d) - ref_p).max() <= 1e-11
+    assert np.array_equal(d.cpu().numpy(), w)
