@@ -130,10 +130,12 @@ struct td1c_ctx {
   // cn_dt / 2, the series terms and the convergence flag
   double cn_dt = 0.0;
   int cn_maxcyc = 20;
-  // terms that the last series of each slot took (pinned, written by the
-  // device), the terms to launch, and how often fewer would have done
+  // terms of each slot's last series and the most of its recent ones (pinned,
+  // written by the device; the latter kept in cn_peak), the terms to launch,
+  // and the series since the window of the recent ones began
   static constexpr int kSeries = 24;
-  int* cn_count_host = nullptr;
+  int* cn_count_host = nullptr;  // [2][kSeries]
+  DevBuf<int> cn_peak;
   int cn_want[kSeries] = {}, cn_low[kSeries] = {}, cn_since = 0;
   double cn_thresh = 1.0e-10;
   int cn_K = 0, cn_npart1 = 0;
@@ -254,6 +256,7 @@ struct td1c_ctx {
     for (auto* b : fm) b->release();
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (cn_count_host) (void)hipHostFree(cn_count_host);
+    cn_peak.release();
     if (cap_stream) (void)hipStreamDestroy(cap_stream);
     for (auto& e : fj)
       if (e) (void)hipEventDestroy(e);
@@ -2059,13 +2062,14 @@ static CnArgs cn_args(td1c_ctx* c, const double* d_lf, double2* wfn) {
 // maxcyc more terms (mode 1) of a series whose first term is enqueued.
 // A captured or recorded step holds every term (the converged ones return
 // at once).  Under stream launches the call enqueues one term more than the
-// longest of the slot's recent series took, as far as their counts have
-// arrived, and k_cn_tail, which forms whatever is still missing: any choice
+// longest of the slot's recent series took (one slot serves series of
+// different lengths: a propagator applies one factor to several vectors of a
+// step), as far as their counts have arrived, and k_cn_tail, which forms whatever is still missing: any choice
 // gives the same bits, and no call waits for the device.  A converged term
 // costs its three launches (about 9 us), a missing one is formed slowly, so
 // the choice follows an increase at once and a decrease after 64 series, and
-// the host waits for the device once in 16 series, so that the counts it has
-// are of a step or two before.  The first series of a slot (of new factors)
+// the host waits for the device once in 16 series, and in the one after an
+// increase, so that the counts it has are of a step or two before.  The first series of a slot (of new factors)
 // reads the count back after the second term and every two terms after.
 static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& obp, int maxcyc, int slot, hipStream_t s) {
   CnArgs a = a0;
@@ -2079,33 +2083,38 @@ static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& ob
   }
   if (slot < 0 || slot >= td1c_ctx::kSeries) slot = 0;
   if (!c->cn_count_host)
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), td1c_ctx::kSeries * sizeof(int)));
-  volatile int* count = c->cn_count_host + slot;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), 2 * td1c_ctx::kSeries * sizeof(int)));
+  if (!c->cn_peak.p) HIP_TRY(c->cn_peak.alloc(td1c_ctx::kSeries));
+  volatile int *count = c->cn_count_host + slot, *count_peak = count + td1c_ctx::kSeries;
+  auto tail = [&](int k, int maxk, bool fresh) {
+    launch_cn_tail(a, obp, c->ob_lc, k, maxk, const_cast<int*>(count), const_cast<int*>(count_peak), c->cn_peak.p + slot,
+                   fresh ? 1 : 0, s);
+  };
   if (c->cn_want[slot] == 0) {
-    *count = 0;
+    *count = *count_peak = 0;
     for (int k = 0; k < maxcyc;) {
       const int chunk = k == 0 ? 1 : 2;
       for (int j = 0; j < chunk && k < maxcyc; ++j) term(++k);
-      launch_cn_tail(a, obp, c->ob_lc, k, k, c->cn_count_host + slot, s);  // the test alone
+      tail(k, k, true);  // the test alone
       HIP_TRY(hipStreamSynchronize(s));
       if (*count >= 0) break;
     }
-    const int n = *count;
-    c->cn_want[slot] = (n >= 0 ? n : -1 - n) + 1;
+    c->cn_want[slot] = *count_peak + 1;
+    c->cn_low[slot] = maxcyc > 0 ? 0 : 64;  // (no launch has set the peak)
     return 0;
   }
   if (++c->cn_since >= 16) {
     HIP_TRY(hipStreamSynchronize(s));
     c->cn_since = 0;
   }
-  const int n = *count, need = (n >= 0 ? n : -1 - n) + 1;
-  if (need >= c->cn_want[slot] || ++c->cn_low[slot] >= 64) {
-    c->cn_want[slot] = need;
-    c->cn_low[slot] = 0;
-  }
+  const int need = *count_peak + 1;
+  const bool fresh = ++c->cn_low[slot] >= 64;
+  if (need > c->cn_want[slot]) c->cn_since = 16;
+  if (need > c->cn_want[slot] || fresh) c->cn_want[slot] = need;
+  if (fresh) c->cn_low[slot] = 0;
   const int m = std::min(maxcyc, c->cn_want[slot]);
   for (int k = 1; k <= m; ++k) term(k);
-  launch_cn_tail(a, obp, c->ob_lc, m, maxcyc, c->cn_count_host + slot, s);
+  tail(m, maxcyc, fresh);
   return 0;
 }
 

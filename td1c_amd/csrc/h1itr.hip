@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(BS) k_cn_bridge(const CnArgs a, int mode) {
 // interior row, every dynamical orbital in groups of kCnGroup: x_I = G_e y_I
 // - W_l x_left - W_r x_right with the row of G_e loaded once into registers
 // for all orbitals, into x and the state, and the block's share of sum
-// |x|^2 into the partial sums that k_cn_check adds (the test at the top of
+// |x|^2 into the partial sums that cn_check_body adds (the test at the top of
 // the next cycle of h1itr_prop.F90:75-99).
 template <int NI>
 __device__ __forceinline__ void cn_interior_body(const CnArgs& a, int mode, int epb, int nchunk, const Blk bk) {
@@ -307,14 +307,16 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc
 // of the last term launched, and while it fails the further terms, the blocks
 // of their three launches walked one after the other (the same bits; slow, and
 // reached only when a series grows by more than the terms the host added to
-// what the previous ones took).  The number of terms (-1 - it when the series
-// has not converged) goes to pinned host memory for the next call's choice, so
-// that no call waits for the device: the test as a launch, the copy of its flag
+// what the recent ones took).  The number of terms (-1 - it when the series
+// has not converged) and the most terms of the series since the last one with
+// `fresh` set (kept in *peak) go to pinned host memory for the next calls'
+// choice, so that no call waits for the device: the test as a launch, the copy of its flag
 // and the wait took about 35 us per half step (8 steps of a He problem on 799
 // points 4.56 -> 3.97 ms).
 template <int NM>
 __global__ void __launch_bounds__(256) k_cn_tail(const CnArgs a, const OneBodyElArgs e, int lc, int term0, int maxcyc,
-                                                 int epb, int nchunk, int* __restrict__ count) {
+                                                 int epb, int nchunk, int* __restrict__ count,
+                                                 int* __restrict__ count_peak, int* __restrict__ peak, int fresh) {
   const int nd = a.nfun - a.nfcore;
   int last = a.flag[1];
   bool done = a.flag[0] != 0;
@@ -352,18 +354,22 @@ __global__ void __launch_bounds__(256) k_cn_tail(const CnArgs a, const OneBodyEl
       last = term;
     }
   }
-  if (threadIdx.x == 0) *count = done ? last : -1 - last;
+  if (threadIdx.x == 0) {
+    *count = done ? last : -1 - last;
+    *count_peak = *peak = fresh ? last : max(*peak, last);
+  }
 }
 
 void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
-                    hipStream_t s) {
+                    int* count_peak, int* peak, int fresh, hipStream_t s) {
   const int epb = std::min(32, kCnInteriorThreads / a.ni), nchunk = (a.nfe + epb - 1) / epb;
   OneBodyElArgs e = ob;
   e.cn = 2;
   cn_check_args(a, e);
   lc = std::max(1, std::min(lc, a.L1));
   auto go = [&](auto k) {
-    hipLaunchKernelGGL(k, dim3(1), dim3(256), 0, s, a, e, lc, term0, maxcyc, epb, nchunk, count);
+    hipLaunchKernelGGL(k, dim3(1), dim3(256), 0, s, a, e, lc, term0, maxcyc, epb, nchunk, count, count_peak, peak,
+                       fresh);
   };
   if (a.n == 20) go(k_cn_tail<20>);
   else if (a.n <= 16) go(k_cn_tail<16>);

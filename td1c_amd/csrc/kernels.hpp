@@ -57,7 +57,7 @@ struct OneBodyElArgs {
   double2 cv;
   const int* stop;
   // cn = 2 with chk_part set: first the convergence test of the previous
-  // term (the sum of its chk_n block partial norms in k_cn_check's order,
+  // term (the sum of its chk_n block partial norms in cn_check_body's order,
   // rms over chk_nfun orbitals below chk_thresh): when it passes, chk_flag
   // is set (by one block) and the launch returns
   const double* chk_part;
@@ -105,9 +105,10 @@ int cn_interior_blocks(const CnArgs& a);
 void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc, int mode, hipStream_t s);
 // after term0 later terms: the convergence test of the last one and the terms
 // still missing up to maxcyc; the number n formed goes to *count (host
-// memory), -1 - n when the series has not converged
+// memory), -1 - n when the series has not converged; the largest n since the
+// launch with `fresh` set goes to *peak (device) and *count_peak (host)
 void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
-                    hipStream_t s);
+                    int* count_peak, int* peak, int fresh, hipStream_t s);
 
 struct PoissonArgs {
   int nr, n, nfe, ni, L2, npair;
@@ -261,7 +262,7 @@ struct LegendreJob {
   FcPhaseJob fc;
 };
 inline int pad_cols(int C) { return (C + 31) / 32 * 32; }
-// mode 0: plain input; 1: pair products (theta -> l).  path: 0 by grid size,
+// mode 0: plain input; 1: pair products (theta -> l).  path: 0 by the number of columns,
 // 1 the vector form, 2 the matrix-core (MFMA) form; tvar: rows per block of
 // the matrix-core form (0: 32, else 16; same bits)
 template <class TI, class TO>

@@ -31,8 +31,8 @@ namespace td1c {
 // the autotuner; every shape gives the same bits.  NM = n for n = 20, else an
 // upper bound of n (16, 24, 32): the rows are padded with zeros.
 // ---------------------------------------------------------------------------
-// The convergence test of a clh1itr term (k_cn_check's arithmetic) in a
-// block of BS threads: the partial sums added by 256 lanes in k_cn_check's
+// The convergence test of a clh1itr term (cn_check_body's arithmetic) in a
+// block of BS threads: the partial sums added by 256 lanes in cn_check_body's
 // order (lane v takes v, v + 256, ...; a butterfly in each wave of 64
 // lanes; the four wave sums in order), so that every block size decides
 // with the same bits.  Every thread of the block gets the result.
