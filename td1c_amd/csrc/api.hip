@@ -205,6 +205,18 @@ struct td1c_ctx {
     int tab[3];
   };
   std::vector<std::unique_ptr<EtdTab>> etd_tabs;
+  std::vector<std::unique_ptr<EtdTab>> etd_spare;  // during a generation only: buffers of the tables it replaces
+  // the operator T_l and the scratch for making the tables
+  DevBuf<double> etd_kb;  // radk, radk0
+  DevBuf<double2> etd_td, etd_vfc, etd_sch;
+  DevBuf<int> etd_err;
+  void release_spare() {
+    for (auto& t : etd_spare) {
+      DevBuf<double2>* e[] = {&t->G, &t->Wl, &t->Wr, &t->pa, &t->pg, &t->binv};
+      for (auto* b : e) b->release();
+    }
+    etd_spare.clear();
+  }
   EtdRat etd[7];
   int etd_scheme = 0;  // 1 cletdrb, 2 cletdrk4, 3 cllawrk, 4 clexpab
   // clexpab: the inverse Taylor matrix (column-major), steps since gen, the
@@ -261,10 +273,13 @@ struct td1c_ctx {
     for (auto& e : fj)
       if (e) (void)hipEventDestroy(e);
     if (clock.p) (void)hipFree(clock.p);
-    for (auto& t : etd_tabs) {
-      DevBuf<double2>* e[] = {&t->G, &t->Wl, &t->Wr, &t->pa, &t->pg, &t->binv};
-      for (auto* b : e) b->release();
-    }
+    for (auto& t : etd_tabs) etd_spare.push_back(std::move(t));
+    release_spare();
+    etd_kb.release();
+    etd_td.release();
+    etd_vfc.release();
+    etd_sch.release();
+    etd_err.release();
     etd_buf.release();
     chk_buf.release();
     chk_ov.release();
@@ -2554,11 +2569,6 @@ int etd_set(td1c_ctx* c, int r, double dfac, const double* num, int dimn, const 
   R.numer_limit = d2(nl);
   R.denom_limit = d2(den);
   R.coeff_limit = d2(nl / den);
-  auto up = [](DevBuf<double2>& b, const std::vector<double>& v) -> hipError_t {
-    hipError_t e = b.alloc(std::max<size_t>(v.size() / 2, 1));
-    if (e != hipSuccess || v.empty()) return e;
-    return hipMemcpy(b.p, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice);
-  };
   for (int i = 0; i < 3; ++i) {
     R.tab[i] = -1;
     if (i >= dimd || !(std::abs(cd1[i]) > thresh)) continue;
@@ -2566,22 +2576,38 @@ int etd_set(td1c_ctx* c, int r, double dfac, const double* num, int dimn, const 
     for (size_t t = 0; t < c->etd_tabs.size(); ++t)
       if (c->etd_tabs[t]->fre == f.real() && c->etd_tabs[t]->fim == f.imag()) R.tab[i] = (int)t;
     if (R.tab[i] >= 0) continue;
-    CnTables T;
-    std::string err;
-    if (!build_cn(S, c->v2jfc_h.empty() ? nullptr : c->v2jfc_h.data(), f.real(), f.imag(), T, err))
-      return fail(-5, err);
-    auto tab = std::make_unique<td1c_ctx::EtdTab>();
-    HIP_TRY(up(tab->G, T.G));
-    HIP_TRY(up(tab->Wl, T.Wl));
-    HIP_TRY(up(tab->Wr, T.Wr));
-    HIP_TRY(up(tab->pa, T.pa));
-    HIP_TRY(up(tab->pg, T.pg));
-    HIP_TRY(up(tab->binv, T.binv));
-    tab->K = T.K;
-    tab->fre = f.real();
-    tab->fim = f.imag();
+    std::unique_ptr<td1c_ctx::EtdTab> tab;
+    if (!c->etd_spare.empty()) {  // the last factors' buffers: all sizes are the context's
+      tab = std::move(c->etd_spare.back());
+      c->etd_spare.pop_back();
+    } else {
+      tab = std::make_unique<td1c_ctx::EtdTab>();
+    }
+    const int ni = S.n - 1, nbr = S.nfe - 1;
+    int K = 0;
+    while ((1 << K) < nbr) ++K;
+    const size_t L1 = S.L1, np = L1 * std::max(K, 1) * nbr;
+    const std::pair<DevBuf<double2>*, size_t> bufs[] = {{&tab->G, L1 * S.nfe * ni * ni}, {&tab->Wl, L1 * S.nr},
+                                                        {&tab->Wr, L1 * S.nr}, {&tab->pa, np}, {&tab->pg, np},
+                                                        {&tab->binv, L1 * nbr}};
+    td1c_ctx::EtdTab& T = *tab;
     R.tab[i] = (int)c->etd_tabs.size();
     c->etd_tabs.push_back(std::move(tab));
+    for (auto& [buf, len] : bufs)
+      if (!buf->p) HIP_TRY(buf->alloc(len));
+    T.K = K;
+    T.fre = f.real();
+    T.fim = f.imag();
+    CnGenArgs g{};
+    g.radk = c->etd_kb.p; g.radk0 = c->etd_kb.p + S.radk.size();
+    g.tdiag = c->etd_td.p; g.v2jfc = c->v2jfc_h.empty() ? nullptr : c->etd_vfc.p;
+    g.fac = d2(f);
+    g.G = T.G.p; g.Wl = T.Wl.p; g.Wr = T.Wr.p; g.pa = T.pa.p; g.pg = T.pg.p; g.binv = T.binv.p;
+    g.sch = c->etd_sch.p; g.pcr = c->etd_sch.p + L1 * S.nfe * 3;
+    g.err = c->etd_err.p;
+    g.n = S.n; g.nr = S.nr; g.nfe = S.nfe; g.L1 = S.L1; g.K = K;
+    launch_cn_generate(g, nullptr);
+    HIP_TRY(hipGetLastError());
   }
   return 0;
 }
@@ -2638,12 +2664,30 @@ int etd_generate(td1c_ctx* c, int scheme, double dt, int rosen, int maxcyc, doub
   if (!(dt != 0.0) || !std::isfinite(dt)) return fail(-1, std::string(name) + " needs a finite nonzero dtime");
   if (maxcyc < 0 || !(thresh >= 0.0)) return fail(-1, "bad maxcyc or thresh");
   if (c->etd_buf.p) HIP_TRY(hipDeviceSynchronize());  // earlier steps may still read the old tables
-  for (auto& t : c->etd_tabs) {
-    DevBuf<double2>* e[] = {&t->G, &t->Wl, &t->Wr, &t->pa, &t->pg, &t->binv};
-    for (auto* b : e) b->release();
-  }
-  c->etd_tabs.clear();
   c->etd_ready = false;
+  for (auto& t : c->etd_tabs) c->etd_spare.push_back(std::move(t));
+  c->etd_tabs.clear();
+  struct SpareGuard {  // the buffers that the new set does not take are given back
+    td1c_ctx* c;
+    ~SpareGuard() { c->release_spare(); }
+  } guard{c};
+  if (scheme != 3) {
+    if (!c->etd_kb.p) {
+      std::vector<double> kb(S.radk);
+      kb.insert(kb.end(), S.radk0.begin(), S.radk0.end());
+      HIP_TRY(c->etd_kb.upload(kb));
+    }
+    auto up = [](DevBuf<double2>& b, const std::vector<double>& v) -> hipError_t {
+      if (!b.p)
+        if (hipError_t e = b.alloc(v.size() / 2); e != hipSuccess) return e;
+      return hipMemcpy(b.p, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice);
+    };
+    if (!c->etd_td.p) HIP_TRY(up(c->etd_td, S.tdiag));
+    if (!c->v2jfc_h.empty()) HIP_TRY(up(c->etd_vfc, c->v2jfc_h));
+    if (!c->etd_sch.p) HIP_TRY(c->etd_sch.alloc((size_t)S.L1 * (3 * S.nfe + 6 * (S.nfe - 1))));
+    if (!c->etd_err.p) HIP_TRY(c->etd_err.alloc(1));
+    HIP_TRY(hipMemset(c->etd_err.p, 0, sizeof(int)));
+  }
   for (int& w : c->cn_want) w = 0;
   if (scheme == 1) {
     const int fam[kEtdRats] = {0, 0, 1, 1, 2, 2, 3};
@@ -2687,6 +2731,12 @@ int etd_generate(td1c_ctx* c, int scheme, double dt, int rosen, int maxcyc, doub
     c->etd[kF0].rk = make_double2(dt / 6.0, 0.0);
     c->etd[kF1].rk = make_double2(dt / 3.0, 0.0);
     c->etd[kF2].rk = make_double2(dt / 6.0, 0.0);
+  }
+  if (scheme != 3) {
+    int err = 0;  // the copy also waits for the tables: any stream may read them afterwards
+    HIP_TRY(hipMemcpy(&err, c->etd_err.p, sizeof(int), hipMemcpyDeviceToHost));
+    if (err & 1) return fail(-5, "singular element block of the Crank-Nicolson operator");
+    if (err & 2) return fail(-5, "Crank-Nicolson bridge system: cyclic reduction met a zero pivot");
   }
   if (int rc = cn_buffers(c)) return rc;
   const size_t so = (size_t)c->nbas * S.nfun, sz = so + S.lcic;

@@ -523,6 +523,184 @@ void launch_cn_interior_grouped(const void* recs, const int2* items, const int* 
                      static_cast<const CnRec*>(recs), items, jobs, sh);
 }
 
+// 1 / z with the parts scaled by the larger one (Smith's division).
+__device__ __forceinline__ double2 cinv(double2 z) {
+  if (fabs(z.x) >= fabs(z.y)) {
+    const double q = z.y / z.x, d = 1.0 / (z.x + z.y * q);
+    return make_double2(d, -q * d);
+  }
+  const double q = z.x / z.y, d = 1.0 / (z.x * q + z.y);
+  return make_double2(q * d, -d);
+}
+
+// (1 + fac T_l)(i, j) at interior points of the grid
+__device__ __forceinline__ double2 cn_entry(const CnGenArgs& a, int l, int i, int j) {
+  if (i == j) {
+    double2 t = a.tdiag[(size_t)l * a.nr + i];
+    if (a.v2jfc) t = cadd(t, a.v2jfc[i]);
+    t = cmul(a.fac, t);
+    return make_double2(1.0 + t.x, t.y);
+  }
+  if (abs(i - j) > a.n) return make_double2(0.0, 0.0);
+  const double* kb = l == 0 ? a.radk : a.radk0;
+  return cscale(a.fac, kb[(size_t)(2 * a.n + 1) * (i + 1) + (a.n + j - i)]);
+}
+
+// The element part of the tables, one wavefront per (element, l): the block in
+// LDS is inverted in place by Gauss-Jordan with row pivoting, FP64, in the
+// order of build_cn's elimination.  The tables of an exponential propagator are
+// 15 such sets; made on the host, one after the other, they were half of a
+// 100-cycle imaginary-time relaxation (Ne, 60 elements, 16 l values: 336 ms
+// with them, 156 ms with these kernels).  A block's 19 steps are latency; all
+// blocks of a set are in flight at once.
+__global__ void __launch_bounds__(64) k_cn_gen_elem(CnGenArgs a) {
+  extern __shared__ double2 cg_lds[];
+  const int n = a.n, ni = n - 1, e = blockIdx.x, l = blockIdx.y, t = threadIdx.x, base = e * n;
+  double2 *sA = cg_lds, *sF = sA + ni * ni, *sC = sF + ni, *sW = sC + 2 * ni;  // sC, sW: left, right
+  __shared__ int sPiv[32];
+  for (int q = t; q < ni * ni; q += 64) sA[q] = cn_entry(a, l, base + q / ni, base + q % ni);
+  const int bl = e >= 1 ? base - 1 : -1, br = e <= a.nfe - 2 ? base + n - 1 : -1;
+  if (t < ni) {
+    sC[t] = bl >= 0 ? cn_entry(a, l, bl, base + t) : make_double2(0.0, 0.0);
+    sC[ni + t] = br >= 0 ? cn_entry(a, l, br, base + t) : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+  for (int c = 0; c < ni; ++c) {
+    // first row of the largest |re| + |im| at or below the diagonal
+    double best = -1.0;
+    int piv = c;
+    if (t >= c && t < ni) {
+      const double2 z = sA[t * ni + c];
+      best = fabs(z.x) + fabs(z.y);
+      piv = t;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      const double ob = __shfl_xor(best, o, 64);
+      const int op = __shfl_xor(piv, o, 64);
+      if (ob > best || (ob == best && op < piv)) {
+        best = ob;
+        piv = op;
+      }
+    }
+    piv = __shfl(piv, 0, 64);  // one row for all lanes, also among NaN
+    const double2 p = sA[piv * ni + c];
+    double2 x = make_double2(0.0, 0.0), y = x;
+    if (t < ni) {
+      x = sA[piv * ni + t];
+      y = sA[c * ni + t];
+    }
+    __syncthreads();
+    if (t == 0) {
+      sPiv[c] = piv;
+      if (p.x == 0.0 && p.y == 0.0) atomicOr(a.err, 1);
+    }
+    const double2 d = cinv(p);
+    if (t < ni) {
+      sA[piv * ni + t] = y;
+      sA[c * ni + t] = t == c ? d : cmul(x, d);
+    }
+    __syncthreads();
+    if (t < ni) sF[t] = sA[t * ni + c];
+    __syncthreads();
+    for (int q = t; q < ni * ni; q += 64) {
+      const int r = q / ni, k = q % ni;
+      if (r == c) continue;
+      const double2 f = sF[r];
+      double2 z = k == c ? make_double2(0.0, 0.0) : sA[q];
+      cfma(z, make_double2(-f.x, -f.y), sA[c * ni + k]);
+      sA[q] = z;
+    }
+    __syncthreads();
+  }
+  if (t < ni)  // the row exchanges undone as column exchanges
+    for (int c = ni - 1; c >= 0; --c) {
+      const int p = sPiv[c];
+      const double2 z = sA[t * ni + c];
+      sA[t * ni + c] = sA[t * ni + p];
+      sA[t * ni + p] = z;
+    }
+  __syncthreads();
+  double2* G = a.G + ((size_t)l * a.nfe + e) * ni * ni;
+  for (int q = t; q < ni * ni; q += 64) G[q] = sA[(q % ni) * ni + q / ni];  // [k][i] = G(i, k)
+  if (t < ni) {
+    double2 wl = make_double2(0.0, 0.0), wr = wl;
+    for (int b = 0; b < ni; ++b) {
+      cfma(wl, sA[t * ni + b], sC[b]);
+      cfma(wr, sA[t * ni + b], sC[ni + b]);
+    }
+    sW[t] = wl;
+    sW[ni + t] = wr;
+    a.Wl[(size_t)l * a.nr + base + t] = wl;
+    a.Wr[(size_t)l * a.nr + base + t] = wr;
+  }
+  if (t == 0 && br >= 0) a.Wl[(size_t)l * a.nr + br] = a.Wr[(size_t)l * a.nr + br] = make_double2(0.0, 0.0);
+  __syncthreads();
+  if (t < 3) {  // the bridge corrections (left, left), (right, right), (left, right)
+    const double2 *u = sC + (t == 1 ? ni : 0), *v = sW + (t == 0 ? 0 : ni);
+    double2 z = make_double2(0.0, 0.0);
+    for (int b = 0; b < ni; ++b) cfma(z, u[b], v[b]);
+    a.sch[((size_t)l * a.nfe + e) * 3 + t] = z;
+  }
+}
+
+// The bridge part, one block per l: the symmetric tridiagonal Schur system and
+// its parallel cyclic reduction factors; the six work rows stay in L2.
+__global__ void __launch_bounds__(256) k_cn_gen_bridge(CnGenArgs a) {
+  const int n = a.n, nb = a.nfe - 1, l = blockIdx.x, K = a.K;
+  double2* row = a.pcr + (size_t)l * 6 * nb;
+  const double2* sch = a.sch + (size_t)l * a.nfe * 3;
+  const double2 zero = make_double2(0.0, 0.0);
+  auto off = [&](int k) {  // between bridges k and k + 1
+    const int gi = (k + 1) * n - 1;
+    return csub(cn_entry(a, l, gi, gi + n), sch[3 * (k + 1) + 2]);
+  };
+  for (int i = threadIdx.x; i < nb; i += 256) {
+    const int gi = (i + 1) * n - 1;
+    row[i] = i > 0 ? off(i - 1) : zero;
+    row[nb + i] = csub(csub(cn_entry(a, l, gi, gi), sch[3 * i + 1]), sch[3 * (i + 1)]);
+    row[2 * nb + i] = i + 1 < nb ? off(i) : zero;
+  }
+  __syncthreads();
+  int cur = 0;
+  for (int k = 0, h = 1; k < K; ++k, h *= 2, cur ^= 1) {
+    const double2 *A = row + (size_t)cur * 3 * nb, *B = A + nb, *C = B + nb;
+    double2* N = row + (size_t)(cur ^ 1) * 3 * nb;
+    for (int i = threadIdx.x; i < nb; i += 256) {
+      double2 al = zero, ga = zero, na = zero, nc = zero, b = B[i];
+      if (i - h >= 0) {
+        al = cmul(A[i], cinv(B[i - h]));
+        al = make_double2(-al.x, -al.y);
+        na = cmul(al, A[i - h]);
+        cfma(b, al, C[i - h]);
+      }
+      if (i + h < nb) {
+        ga = cmul(C[i], cinv(B[i + h]));
+        ga = make_double2(-ga.x, -ga.y);
+        nc = cmul(ga, C[i + h]);
+        cfma(b, ga, A[i + h]);
+      }
+      a.pa[((size_t)l * K + k) * nb + i] = al;
+      a.pg[((size_t)l * K + k) * nb + i] = ga;
+      N[i] = na;
+      N[nb + i] = b;
+      N[2 * nb + i] = nc;
+    }
+    __syncthreads();
+  }
+  const double2* B = row + (size_t)cur * 3 * nb + nb;
+  for (int i = threadIdx.x; i < nb; i += 256) {
+    if (!(hypot(B[i].x, B[i].y) > 1e-300)) atomicOr(a.err, 2);
+    a.binv[(size_t)l * nb + i] = cinv(B[i]);
+  }
+}
+
+void launch_cn_generate(const CnGenArgs& a, hipStream_t s) {
+  const int ni = a.n - 1;
+  const size_t lds = (size_t)(ni * ni + 5 * ni) * sizeof(double2);
+  hipLaunchKernelGGL(k_cn_gen_elem, dim3(a.nfe, a.L1), dim3(64), lds, s, a);
+  hipLaunchKernelGGL(k_cn_gen_bridge, dim3(a.L1), dim3(256), 0, s, a);
+}
+
 bool launch_batch_h1itr(const LaunchRec& p, const void* recs, const BatchMap& map, int grid, size_t lds,
                         hipStream_t s, bool dry) {
   const CnRec* r = static_cast<const CnRec*>(recs);

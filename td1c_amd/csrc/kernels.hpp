@@ -599,6 +599,20 @@ struct CnShared {
   int epb;      // elements per block (every member's)
   SeriesGate gate;
 };
+// Element Schur tables of 1 + fac T_l made on the device (build_cn's numbers):
+// radk / radk0 (band rows of 2 n + 1, l = 0 / l >= 1), tdiag[L1][nr], v2jfc[nr]
+// or null; scratch: sch[L1][nfe][3], pcr[L1][6][nb]; err gets bit 0 for a
+// singular element block, bit 1 for a zero bridge pivot.
+struct CnGenArgs {
+  const double *radk, *radk0;
+  const double2 *tdiag, *v2jfc;
+  double2 fac;
+  double2 *G, *Wl, *Wr, *pa, *pg, *binv;
+  double2 *sch, *pcr;
+  int* err;
+  int n, nr, nfe, L1, K;
+};
+void launch_cn_generate(const CnGenArgs& a, hipStream_t s);
 void launch_cn_interior_grouped(const void* recs, const int2* items, const int* jobs, int njobs, const CnShared& sh,
                                 hipStream_t s);
 // sites whose blocks return at once for a converged member (the later terms

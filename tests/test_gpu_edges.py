@@ -101,3 +101,33 @@ def test_observables_in_place(gpu_lib, igauge, nact):
     assert np.abs(hp.dipole3(lf, d) - ref).max() <= 1e-11 * scale
     assert np.abs(hp.ipx(2, 4.0, lf, d) - ref_p).max() <= 1e-11
     assert np.array_equal(d.cpu().numpy(), w)
+
+
+# the factors of the exponential propagators, made on the device: one to 31
+# interior points per element, 2 elements (one bridge, no reduction step) to
+# 161 (the most), with and without a frozen core; made again in
+# the buffers of another step size's and another scheme's factors
+@pytest.mark.parametrize("ndvr,nfe,nfc", [(2, 2, 0), (2, 161, 1), (5, 24, 0), (20, 2, 1), (20, 9, 0), (32, 5, 1)])
+def test_etd_factors(gpu_lib, ndvr, nfe, nfc):
+    import torch
+
+    prob = Problem(nfe=nfe, ndvr=ndvr, rmax=max(9.0, 0.2 * nfe), lmax1=2, lmax2=4, znuc=4.0, nfcore1=nfc, ndcore=2 - nfc,
+                   nel_alpha=2, nel_beta=2, lval=[0, 0], igauge=1, isplit=1)
+    o = Oracle(prob)
+    w = C.smooth_wfn_for(prob, o.lcic)
+    o.set_wfn0(w)
+    o.etdrb_gen(0.01)
+    lf = np.zeros(54)
+    lf[:27] = np.tile(C.LF_VEL, 3)
+    ref = o.etdrb_step(lf, w.copy(), apply_mask=False)
+    hp = td1c_amd.HProd(prob)
+    hp.set_wfn0(w)
+    td1c_amd.ETDRB(hp, 0.02)
+    for again in range(2):
+        etd = td1c_amd.ETDRB(hp, 0.01)
+        d = hp.to_device(w)
+        etd.prop(d, lfields=lf, apply_mask=False)
+        torch.cuda.synchronize()
+        assert np.linalg.norm(d.cpu().numpy() - ref) < 1e-10 * np.linalg.norm(ref)
+        td1c_amd.ETDRK4(hp, 0.02)
+    hp.close()
