@@ -116,6 +116,7 @@ def kernel_bytes(name: str, s: dict, cm: int = 16) -> float:
     nr, L1, L2, nl = s["nr"], s["L1"], s["L2"], s["nlat"]
     nf, nd, npair, nfc = s["nfun"], s["ndyn"], s["npair"], s["nfcore"]
     nb, ng, c = nr * L1, nr * nl, 16
+    nv = nd if s["nactpair"] > 0 else 0  # v2 rows: zero, and not formed, without active orbitals
     table = {
         # with the velocity-gauge frozen-core phase carried by the same launch
         "l2theta": nd * (nb * c + ng * cm) + nfc * ng * (c + cm),
@@ -125,13 +126,13 @@ def kernel_bytes(name: str, s: dict, cm: int = 16) -> float:
         "poisson_bridge": npair * L2 * nr * cm,
         "poisson_interior": 2 * npair * L2 * nr * cm,
         "pair_L2theta": npair * (L2 * nr + ng) * cm,
-        "mfprod": (nf * ng + npair * ng + 2 * nd * ng) * cm,
-        "theta2l_mf": 2 * nd * (ng * cm + nb * c),
-        "gram_l": (nf + nfc + 4 * nd) * nb * c,
+        "mfprod": (nf * ng + npair * ng + (nd + nv) * ng) * cm,
+        "theta2l_mf": (nd + nv) * (ng * cm + nb * c),
+        "gram_l": (nf + nfc + 2 * nd + nv + (nd if nfc else 0)) * nb * c,
         "gram_pair": 2 * s["nactpair"] * L2 * nr * cm,
         # k: read h01, g, v2, orb of nf and all orbitals for X; acc r+w; w0 r; next w; k w; earlier k r
-        "dtorb_rk": (nd * 3 + nf + nf * 2 + nf + nf + nf + 1.5 * nf) * nb * c,
-        "dtorb": (nd * 3 + nf + nf) * nb * c,
+        "dtorb_rk": (nd * 2 + nv + nf + nf * 2 + nf + nf + nf + 1.5 * nf) * nb * c,
+        "dtorb": (nd * 2 + nv + nf + nf) * nb * c,
         "island_a": 0.0,
         "island_b": 0.0,
     }
@@ -140,15 +141,16 @@ def kernel_bytes(name: str, s: dict, cm: int = 16) -> float:
 
 def kernel_flops(name: str, s: dict) -> float:
     """Arithmetic of one launch (real flops; a complex-by-real multiply-add
-    is 4): the Legendre transforms on the matrix cores and the Poisson
-    element products."""
+    is 4): the Legendre transforms on the matrix cores (half of the plain
+    product by the mirror symmetry of the theta grid) and the Poisson element
+    products."""
     nr, L1, L2, nl = s["nr"], s["L1"], s["L2"], s["nlat"]
     nd, npair, nfc = s["ndyn"], s["npair"], s["nfcore"]
     table = {
-        "l2theta": 4.0 * nr * L1 * nl * (nd + nfc),
-        "pair_theta2L": 4.0 * nr * nl * L2 * npair + 6.0 * nr * nl * npair,
-        "pair_L2theta": 4.0 * nr * L2 * nl * npair,
-        "theta2l_mf": 2 * 4.0 * nr * nl * L1 * nd,
+        "l2theta": 2.0 * nr * L1 * nl * (nd + nfc),
+        "pair_theta2L": 2.0 * nr * nl * L2 * npair + 6.0 * nr * nl * npair,
+        "pair_L2theta": 2.0 * nr * L2 * nl * npair,
+        "theta2l_mf": (2 if s["nactpair"] > 0 else 1) * 2.0 * nr * nl * L1 * nd,
         "poisson_interior": 4.0 * (s["ndvr"] - 1) * npair * L2 * nr,
     }
     return float(table.get(name, 0.0))

@@ -432,10 +432,10 @@ int td1c_h1itr_gen(td1c_ctx* ctx, double dtime, int maxcyc, double thresh);
  * reference evaluates at t + dt/4 (first half step) or t + 3dt/4 (second).
  * The first check of the series (on x_0, norm ~1 per orbital) counts the
  * dynamical orbitals only.  Enqueued on `stream`; td1c_h1itr_gen first.
- * Under stream launches the call reads the series' flag back after the
- * second term and every two terms after (it waits for `stream` to get
- * there) and enqueues no more terms once the series has converged; under
- * graph capture every term is enqueued.  The same holds for the half steps
+ * Under stream launches the call enqueues as many terms as recent series
+ * took and one more, and a last launch forms whatever is still missing; it
+ * waits for `stream` in the first series of new factors and once in 16
+ * series.  Under graph capture every term is enqueued.  The same holds for the half steps
  * of td1c_propagate and the denominator series of the exponential
  * propagators. */
 int td1c_h1itr_prop(td1c_ctx* ctx, const double* lfield, double* d_wfn, void* stream);
@@ -483,8 +483,8 @@ int td1c_batch_propagate(td1c_batch* batch, const td1c_field* fields, int rk_ord
 int td1c_batch_set_graph(td1c_batch* batch, int on);
 
 /* Launch shapes of the batch: the element one-body kernel's elements per
- * block (3, 6, 12) and l values per block, and the register-blocked
- * transform's variant (0: 4 column tiles, 1: 2 column tiles per wavefront);
+ * block (3, 6, 12) and l values per block, and the matrix-core
+ * transform's variant (0: 16 radial rows per block, 1: 8);
  * every choice gives the same bits. */
 int td1c_batch_set_shapes(td1c_batch* batch, int elements_per_block, int l_per_block, int transform_variant);
 
