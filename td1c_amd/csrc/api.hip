@@ -131,12 +131,12 @@ struct td1c_ctx {
   double cn_dt = 0.0;
   int cn_maxcyc = 20;
   // terms of each slot's last series and the most of its recent ones (pinned,
-  // written by the device; the latter kept in cn_peak), the terms to launch,
-  // and the series since the window of the recent ones began
+  // written by the device; the latter kept in cn_peak) and its number, the
+  // terms to launch, and the series since the window of the recent ones began
   static constexpr int kSeries = 24;
-  int* cn_count_host = nullptr;  // [2][kSeries]
+  int* cn_count_host = nullptr;  // [3][kSeries]
   DevBuf<int> cn_peak;
-  int cn_want[kSeries] = {}, cn_low[kSeries] = {}, cn_since = 0;
+  int cn_want[kSeries] = {}, cn_low[kSeries] = {}, cn_seq[kSeries] = {};
   double cn_thresh = 1.0e-10;
   int cn_K = 0, cn_npart1 = 0;
   DevBuf<double2> cnG, cnWl, cnWr, cnPa, cnPg, cnBinv, cn_x, cn_y;
@@ -2082,10 +2082,13 @@ static CnArgs cn_args(td1c_ctx* c, const double* d_lf, double2* wfn) {
 // step), as far as their counts have arrived, and k_cn_tail, which forms whatever is still missing: any choice
 // gives the same bits, and no call waits for the device.  A converged term
 // costs its three launches (about 9 us), a missing one is formed slowly, so
-// the choice follows an increase at once and a decrease after 64 series, and
-// the host waits for the device once in 16 series, and in the one after an
-// increase, so that the counts it has are of a step or two before.  The first series of a slot (of new factors)
-// reads the count back after the second term and every two terms after.
+// the choice follows an increase at once and a decrease after 64 series; once
+// the tail launch had to form terms (Ar grid: some 20 ms each), all terms are
+// launched for 64 series,
+// and the call waits for the count of the slot's last series, a step ago, or
+// of the one before it (half steps, two a step), so that the device has the
+// work of a step meanwhile.  The first series of a slot (of new factors) reads
+// the count back after the second term and every two terms after.
 static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& obp, int maxcyc, int slot, hipStream_t s) {
   CnArgs a = a0;
   auto term = [&](int k) {
@@ -2098,15 +2101,16 @@ static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& ob
   }
   if (slot < 0 || slot >= td1c_ctx::kSeries) slot = 0;
   if (!c->cn_count_host)
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), 2 * td1c_ctx::kSeries * sizeof(int)));
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), 3 * td1c_ctx::kSeries * sizeof(int)));
   if (!c->cn_peak.p) HIP_TRY(c->cn_peak.alloc(td1c_ctx::kSeries));
-  volatile int *count = c->cn_count_host + slot, *count_peak = count + td1c_ctx::kSeries;
+  volatile int *count = c->cn_count_host + slot, *count_peak = count + td1c_ctx::kSeries, *count_seq = count_peak + td1c_ctx::kSeries;
   auto tail = [&](int k, int maxk, bool fresh) {
     launch_cn_tail(a, obp, c->ob_lc, k, maxk, const_cast<int*>(count), const_cast<int*>(count_peak), c->cn_peak.p + slot,
-                   fresh ? 1 : 0, s);
+                   fresh ? 1 : 0, const_cast<int*>(count_seq), c->cn_seq[slot], s);
   };
   if (c->cn_want[slot] == 0) {
     *count = *count_peak = 0;
+    *count_seq = c->cn_seq[slot] = 0;
     for (int k = 0; k < maxcyc;) {
       const int chunk = k == 0 ? 1 : 2;
       for (int j = 0; j < chunk && k < maxcyc; ++j) term(++k);
@@ -2118,15 +2122,17 @@ static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& ob
     c->cn_low[slot] = maxcyc > 0 ? 0 : 64;  // (no launch has set the peak)
     return 0;
   }
-  if (++c->cn_since >= 16) {
-    HIP_TRY(hipStreamSynchronize(s));
-    c->cn_since = 0;
-  }
+  // the count of series seq - lag (at most two are on their way); the query
+  // ends the wait when the stream has nothing left to do, or has failed
+  const int seq = ++c->cn_seq[slot], lag = slot == 0 ? 2 : 1;
+  for (int spin = 1; *count_seq < seq - lag; ++spin)
+    if (spin % 64 == 0 && hipStreamQuery(s) != hipErrorNotReady) break;
   const int need = *count_peak + 1;
   const bool fresh = ++c->cn_low[slot] >= 64;
-  if (need > c->cn_want[slot]) c->cn_since = 16;
-  if (need > c->cn_want[slot] || fresh) c->cn_want[slot] = need;
-  if (fresh) c->cn_low[slot] = 0;
+  const int more = need - c->cn_want[slot];
+  if (more > 0) c->cn_want[slot] = more > 1 ? std::max(maxcyc, need) : need;
+  else if (fresh) c->cn_want[slot] = need;
+  if (fresh || more > 1) c->cn_low[slot] = 0;
   const int m = std::min(maxcyc, c->cn_want[slot]);
   for (int k = 1; k <= m; ++k) term(k);
   tail(m, maxcyc, fresh);

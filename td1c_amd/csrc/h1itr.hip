@@ -308,15 +308,16 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc
 // of their three launches walked one after the other (the same bits; slow, and
 // reached only when a series grows by more than the terms the host added to
 // what the recent ones took).  The number of terms (-1 - it when the series
-// has not converged) and the most terms of the series since the last one with
-// `fresh` set (kept in *peak) go to pinned host memory for the next calls'
-// choice, so that no call waits for the device: the test as a launch, the copy of its flag
+// has not converged), the most terms of the series since the last one with
+// `fresh` set (kept in *peak) and then the series' number go to pinned host
+// memory for the next calls' choice: the test as a launch, the copy of its flag
 // and the wait took about 35 us per half step (8 steps of a He problem on 799
 // points 4.56 -> 3.97 ms).
 template <int NM>
 __global__ void __launch_bounds__(256) k_cn_tail(const CnArgs a, const OneBodyElArgs e, int lc, int term0, int maxcyc,
                                                  int epb, int nchunk, int* __restrict__ count,
-                                                 int* __restrict__ count_peak, int* __restrict__ peak, int fresh) {
+                                                 int* __restrict__ count_peak, int* __restrict__ peak, int fresh,
+                                                 int* __restrict__ count_seq, int seq) {
   const int nd = a.nfun - a.nfcore;
   int last = a.flag[1];
   bool done = a.flag[0] != 0;
@@ -357,11 +358,13 @@ __global__ void __launch_bounds__(256) k_cn_tail(const CnArgs a, const OneBodyEl
   if (threadIdx.x == 0) {
     *count = done ? last : -1 - last;
     *count_peak = *peak = fresh ? last : max(*peak, last);
+    __threadfence_system();
+    *count_seq = seq;
   }
 }
 
 void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
-                    int* count_peak, int* peak, int fresh, hipStream_t s) {
+                    int* count_peak, int* peak, int fresh, int* count_seq, int seq, hipStream_t s) {
   const int epb = std::min(32, kCnInteriorThreads / a.ni), nchunk = (a.nfe + epb - 1) / epb;
   OneBodyElArgs e = ob;
   e.cn = 2;
@@ -369,7 +372,7 @@ void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0,
   lc = std::max(1, std::min(lc, a.L1));
   auto go = [&](auto k) {
     hipLaunchKernelGGL(k, dim3(1), dim3(256), 0, s, a, e, lc, term0, maxcyc, epb, nchunk, count, count_peak, peak,
-                       fresh);
+                       fresh, count_seq, seq);
   };
   if (a.n == 20) go(k_cn_tail<20>);
   else if (a.n <= 16) go(k_cn_tail<16>);

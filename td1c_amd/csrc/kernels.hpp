@@ -106,9 +106,10 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc
 // after term0 later terms: the convergence test of the last one and the terms
 // still missing up to maxcyc; the number n formed goes to *count (host
 // memory), -1 - n when the series has not converged; the largest n since the
-// launch with `fresh` set goes to *peak (device) and *count_peak (host)
+// launch with `fresh` set goes to *peak (device) and *count_peak (host), seq
+// to *count_seq (host) after them
 void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
-                    int* count_peak, int* peak, int fresh, hipStream_t s);
+                    int* count_peak, int* peak, int fresh, int* count_seq, int seq, hipStream_t s);
 
 struct PoissonArgs {
   int nr, n, nfe, ni, L2, npair;
