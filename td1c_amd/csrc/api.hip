@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -130,13 +131,11 @@ struct td1c_ctx {
   // cn_dt / 2, the series terms and the convergence flag
   double cn_dt = 0.0;
   int cn_maxcyc = 20;
-  // terms of each slot's last series and the most of its recent ones (pinned,
-  // written by the device; the latter kept in cn_peak) and its number, the
-  // terms to launch, and the series since the window of the recent ones began
+  // the count that ends a wait for a series (pinned, written by the device)
+  // and the terms of each slot's last series
   static constexpr int kSeries = 24;
-  int* cn_count_host = nullptr;  // [3][kSeries]
-  DevBuf<int> cn_peak;
-  int cn_want[kSeries] = {}, cn_low[kSeries] = {}, cn_seq[kSeries] = {};
+  int* cn_count_host = nullptr;
+  int cn_want[kSeries] = {};
   double cn_thresh = 1.0e-10;
   int cn_K = 0, cn_npart1 = 0;
   DevBuf<double2> cnG, cnWl, cnWr, cnPa, cnPg, cnBinv, cn_x, cn_y;
@@ -268,8 +267,7 @@ struct td1c_ctx {
     for (auto* b : fm) b->release();
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (cn_count_host) (void)hipHostFree(cn_count_host);
-    cn_peak.release();
-    if (cap_stream) (void)hipStreamDestroy(cap_stream);
+      if (cap_stream) (void)hipStreamDestroy(cap_stream);
     for (auto& e : fj)
       if (e) (void)hipEventDestroy(e);
     if (clock.p) (void)hipFree(clock.p);
@@ -2074,21 +2072,35 @@ static CnArgs cn_args(td1c_ctx* c, const double* d_lf, double2* wfn) {
   return a;
 }
 
+// Waits for the count that launch_cn_check sends.  A device that is close
+// behind answers within microseconds, so the pinned word is read in a loop
+// first; after 2 ms (long steps queued ahead) the call sleeps in the stream's
+// own wait, which also reports a stream that failed.
+static int wait_series(td1c_ctx* c, hipStream_t s, int* count) {
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int spin = 1;; ++spin) {
+    *count = __atomic_load_n(c->cn_count_host, __ATOMIC_ACQUIRE);
+    if (*count != kCnPending) return 0;
+    if (spin % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    __builtin_ia32_pause();
+  }
+  HIP_TRY(hipStreamSynchronize(s));
+  *count = __atomic_load_n(c->cn_count_host, __ATOMIC_ACQUIRE);
+  if (*count == kCnPending) return fail(-3, "the series' convergence test did not run");
+  return 0;
+}
+
 // maxcyc more terms (mode 1) of a series whose first term is enqueued.
 // A captured or recorded step holds every term (the converged ones return
-// at once).  Under stream launches the call enqueues one term more than the
-// longest of the slot's recent series took (one slot serves series of
-// different lengths: a propagator applies one factor to several vectors of a
-// step), as far as their counts have arrived, and k_cn_tail, which forms whatever is still missing: any choice
-// gives the same bits, and no call waits for the device.  A converged term
-// costs its three launches (about 9 us), a missing one is formed slowly, so
-// the choice follows an increase at once and a decrease after 64 series; once
-// the tail launch had to form terms (Ar grid: some 20 ms each), all terms are
-// launched for 64 series,
-// and the call waits for the count of the slot's last series, a step ago, or
-// of the one before it (half steps, two a step), so that the device has the
-// work of a step meanwhile.  The first series of a slot (of new factors) reads
-// the count back after the second term and every two terms after.
+// at once).  Under stream launches the call enqueues as many terms as the
+// slot's last series took, then the convergence test, waits for its count and
+// goes on with one term, then two at a time, until the series has converged.
+// Terms after the converged one return at once, so any choice gives the same
+// bits; a term too many costs its three empty launches (about 9 us), a missing
+// one a wait of some 10 us.  Going on without a wait, with the terms still
+// missing formed by one block, took 163 against 25 ms a step where the lengths
+// change (cletdrk4, 9 orbitals, 64 l, 2399 points), and 0.54 against 0.56 where
+// they do not (split2, 1 orbital, 16 l, 799 points).
 static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& obp, int maxcyc, int slot, hipStream_t s) {
   CnArgs a = a0;
   auto term = [&](int k) {
@@ -2100,42 +2112,23 @@ static int enqueue_series(td1c_ctx* c, const CnArgs& a0, const OneBodyElArgs& ob
     return 0;
   }
   if (slot < 0 || slot >= td1c_ctx::kSeries) slot = 0;
-  if (!c->cn_count_host)
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), 3 * td1c_ctx::kSeries * sizeof(int)));
-  if (!c->cn_peak.p) HIP_TRY(c->cn_peak.alloc(td1c_ctx::kSeries));
-  volatile int *count = c->cn_count_host + slot, *count_peak = count + td1c_ctx::kSeries, *count_seq = count_peak + td1c_ctx::kSeries;
-  auto tail = [&](int k, int maxk, bool fresh) {
-    launch_cn_tail(a, obp, c->ob_lc, k, maxk, const_cast<int*>(count), const_cast<int*>(count_peak), c->cn_peak.p + slot,
-                   fresh ? 1 : 0, const_cast<int*>(count_seq), c->cn_seq[slot], s);
-  };
-  if (c->cn_want[slot] == 0) {
-    *count = *count_peak = 0;
-    *count_seq = c->cn_seq[slot] = 0;
-    for (int k = 0; k < maxcyc;) {
-      const int chunk = k == 0 ? 1 : 2;
-      for (int j = 0; j < chunk && k < maxcyc; ++j) term(++k);
-      tail(k, k, true);  // the test alone
-      HIP_TRY(hipStreamSynchronize(s));
-      if (*count >= 0) break;
+  if (!c->cn_count_host) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&c->cn_count_host), sizeof(int)));
+  int k = 0, to = std::max(1, c->cn_want[slot]), step = 1;
+  while (k < maxcyc) {
+    for (to = std::min(to, maxcyc); k < to;) term(++k);
+    __atomic_store_n(c->cn_count_host, kCnPending, __ATOMIC_RELEASE);
+    launch_cn_check(a, c->cn_count_host, s);
+    HIP_TRY(hipGetLastError());
+    int count = 0;
+    if (int rc = wait_series(c, s, &count)) return rc;
+    if (count >= 0) {
+      k = count;
+      break;
     }
-    c->cn_want[slot] = *count_peak + 1;
-    c->cn_low[slot] = maxcyc > 0 ? 0 : 64;  // (no launch has set the peak)
-    return 0;
+    to = k + step;
+    step = 2;
   }
-  // the count of series seq - lag (at most two are on their way); the query
-  // ends the wait when the stream has nothing left to do, or has failed
-  const int seq = ++c->cn_seq[slot], lag = slot == 0 ? 2 : 1;
-  for (int spin = 1; *count_seq < seq - lag; ++spin)
-    if (spin % 64 == 0 && hipStreamQuery(s) != hipErrorNotReady) break;
-  const int need = *count_peak + 1;
-  const bool fresh = ++c->cn_low[slot] >= 64;
-  const int more = need - c->cn_want[slot];
-  if (more > 0) c->cn_want[slot] = more > 1 ? std::max(maxcyc, need) : need;
-  else if (fresh) c->cn_want[slot] = need;
-  if (fresh || more > 1) c->cn_low[slot] = 0;
-  const int m = std::min(maxcyc, c->cn_want[slot]);
-  for (int k = 1; k <= m; ++k) term(k);
-  tail(m, maxcyc, fresh);
+  c->cn_want[slot] = k;
   return 0;
 }
 

@@ -10,11 +10,13 @@
 // same operator is solved by element Schur complement: the interior blocks
 // of each FEDVR element are eliminated with their precomputed inverses and
 // the bridge points form a tridiagonal system solved by cyclic reduction.
-// One term of the series is four launches: the right-hand side (the
-// element one-body kernel in its Crank-Nicolson modes), the bridge pass (one block per orbital row), the interior
-// pass (one block per (l, element chunk), each element inverse read once for
-// every orbital) and the convergence test (one block); every later launch of
-// the half step returns at once after convergence.
+// One term of the series is three launches: the right-hand side (the element
+// one-body kernel in its Crank-Nicolson modes), the bridge pass (one block per
+// orbital row) and the interior pass (one block per (l, element chunk), each
+// element inverse read once for every orbital).  A term's convergence test runs
+// at the start of the next right-hand side, as a launch of its own in a batch
+// and where the host waits for the result; every later launch of the half step
+// returns at once after convergence.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,7 +24,6 @@
 
 #include "devmath.hpp"
 #include "kernels.hpp"
-#include "onebody.hpp"
 
 namespace td1c {
 
@@ -303,81 +304,18 @@ void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc
     hipLaunchKernelGGL((k_cn_interior<0>), grid, dim3(kCnInteriorThreads), 0, s, a, mode, epb, nchunk);
 }
 
-// The end of a series under stream launches, one block: the convergence test
-// of the last term launched, and while it fails the further terms, the blocks
-// of their three launches walked one after the other (the same bits; slow, and
-// reached only when a series grows by more than the terms the host added to
-// what the recent ones took).  The number of terms (-1 - it when the series
-// has not converged), the most terms of the series since the last one with
-// `fresh` set (kept in *peak) and then the series' number go to pinned host
-// memory for the next calls' choice: the test as a launch, the copy of its flag
-// and the wait took about 35 us per half step (8 steps of a He problem on 799
-// points 4.56 -> 3.97 ms).
-template <int NM>
-__global__ void __launch_bounds__(256) k_cn_tail(const CnArgs a, const OneBodyElArgs e, int lc, int term0, int maxcyc,
-                                                 int epb, int nchunk, int* __restrict__ count,
-                                                 int* __restrict__ count_peak, int* __restrict__ peak, int fresh,
-                                                 int* __restrict__ count_seq, int seq) {
-  const int nd = a.nfun - a.nfcore;
-  int last = a.flag[1];
-  bool done = a.flag[0] != 0;
-  if (!done) {
-    OneBodyElArgs r = e;
-    r.chk_part = nullptr;  // (tested here)
-    const int GE = onebody_elements(256, a.n);
-    const int nx = (a.nfe + GE - 1) / GE, ny = (a.L1 + lc - 1) / lc;
-    for (int term = term0 + 1;; ++term) {
-      __syncthreads();
-      if (cn_series_done<256>(e.chk_part, e.chk_n, e.chk_nfun, e.chk_thresh)) {
-        if (threadIdx.x == 0) a.flag[0] = 1;
-        done = true;
-        break;
-      }
-      if (term > maxcyc) break;
-#pragma unroll 1
-      for (int b = 0; b < nx * ny * nd; ++b) {
-        __syncthreads();
-        onebody_el_body<NM, 256, 2>(a.x, a.y, r, lc, Blk{b % nx, (b / nx) % ny, b / (nx * ny), nx, ny, nd});
-      }
-      __threadfence_block();
-#pragma unroll 1
-      for (int b = 0; b < nd * a.L1; ++b) {
-        __syncthreads();
-        cn_bridge_body<256>(a, 1, Blk{b, 0, 0, nd * a.L1, 1, 1});
-      }
-      __threadfence_block();
-#pragma unroll 1
-      for (int b = 0; b < a.L1 * nchunk; ++b) {
-        __syncthreads();
-        cn_interior_body<NM == 20 ? 19 : 0>(a, 1, epb, nchunk, Blk{b, 0, 0, a.L1 * nchunk, 1, 1});
-      }
-      __threadfence_block();
-      last = term;
-    }
-  }
-  if (threadIdx.x == 0) {
-    *count = done ? last : -1 - last;
-    *count_peak = *peak = fresh ? last : max(*peak, last);
-    __threadfence_system();
-    *count_seq = seq;
-  }
+// The convergence test of the last term launched, with its count for the host.
+// The host reads nothing but the count (later launches see the rest in stream
+// order), so that the store needs no release, whose write-back of the L2 would
+// stand before it.
+__global__ void __launch_bounds__(kCnInteriorThreads) k_cn_check(const CnArgs a, int nblk, int* count) {
+  cn_check_body(a, 1, nblk);
+  if (threadIdx.x == 0)
+    __hip_atomic_store(count, a.flag[0] ? a.flag[1] : -1 - a.flag[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
-                    int* count_peak, int* peak, int fresh, int* count_seq, int seq, hipStream_t s) {
-  const int epb = std::min(32, kCnInteriorThreads / a.ni), nchunk = (a.nfe + epb - 1) / epb;
-  OneBodyElArgs e = ob;
-  e.cn = 2;
-  cn_check_args(a, e);
-  lc = std::max(1, std::min(lc, a.L1));
-  auto go = [&](auto k) {
-    hipLaunchKernelGGL(k, dim3(1), dim3(256), 0, s, a, e, lc, term0, maxcyc, epb, nchunk, count, count_peak, peak,
-                       fresh, count_seq, seq);
-  };
-  if (a.n == 20) go(k_cn_tail<20>);
-  else if (a.n <= 16) go(k_cn_tail<16>);
-  else if (a.n <= 24) go(k_cn_tail<24>);
-  else go(k_cn_tail<32>);
+void launch_cn_check(const CnArgs& a, int* count, hipStream_t s) {
+  hipLaunchKernelGGL(k_cn_check, dim3(1), dim3(kCnInteriorThreads), 0, s, a, cn_interior_blocks(a), count);
 }
 
 __global__ void __launch_bounds__(256) k_cn_bridge_batch(const CnRec* __restrict__ recs, const BatchMap map) {

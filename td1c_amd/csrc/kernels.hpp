@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstddef>
 #include <string>
 #include <vector>
@@ -103,13 +104,11 @@ int cn_interior_blocks(const CnArgs& a);
 // ob: the element one-body arguments for the right-hand side, with its launch
 // shape
 void launch_cn_stage(const CnArgs& a, const OneBodyElArgs& ob, int shape, int lc, int mode, hipStream_t s);
-// after term0 later terms: the convergence test of the last one and the terms
-// still missing up to maxcyc; the number n formed goes to *count (host
-// memory), -1 - n when the series has not converged; the largest n since the
-// launch with `fresh` set goes to *peak (device) and *count_peak (host), seq
-// to *count_seq (host) after them
-void launch_cn_tail(const CnArgs& a, const OneBodyElArgs& ob, int lc, int term0, int maxcyc, int* count,
-                    int* count_peak, int* peak, int fresh, int* count_seq, int seq, hipStream_t s);
+// the convergence test of the term just enqueued; the number n of terms formed
+// after the first goes to *count (host memory), -1 - n while the series has not
+// converged
+constexpr int kCnPending = INT_MIN;  // what the host puts there before the launch
+void launch_cn_check(const CnArgs& a, int* count, hipStream_t s);
 
 struct PoissonArgs {
   int nr, n, nfe, ni, L2, npair;

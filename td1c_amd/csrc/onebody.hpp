@@ -1,6 +1,5 @@
-// The element one-body kernel's block (launched from kernels.hip; the tail of
-// a half-step series in h1itr.hip walks its blocks) and the series' convergence
-// test.
+// The element one-body kernel's block (launched from kernels.hip, alone and in
+// batches) and the series' convergence test.
 #pragma once
 
 #include "devmath.hpp"

@@ -189,3 +189,83 @@ def test_split_rejects_what_is_not_provided(gpu_lib):
     hp = td1c_amd.HProd(C.he_small())
     with pytest.raises(RuntimeError):
         hp.h1itr_gen(DT)
+
+
+# fields of one and two terms, of 5 to 12 and of all 20 (unconverged) in turn
+SWITCHED = [0.0, 1e-3, 10.0, 1.0, 100.0, 100.0, 1e-3, 3.0, 1e-3, 100.0]
+
+
+@pytest.mark.parametrize("igauge", [0, 1])
+@pytest.mark.parametrize("ndvr", [5, 17, 20, 32])
+def test_series_of_changing_length(gpu_lib, ndvr, igauge):
+    """Half steps whose series grow and shrink from call to call on one
+    context give the bits that a fresh context gives for the same state and
+    field, and the oracle's (1e-11)."""
+    import torch
+    import td1c_amd
+    from oracle.oracle import Oracle
+
+    prob = C.Problem(nfe=7, ndvr=ndvr, rmax=14.0, lmax1=5, lmax2=10, znuc=5.0, nfcore1=1, ndcore=2, nel_alpha=3,
+                     nel_beta=3, mval=[0, 0, 1], lval=[0, 0, 1], igauge=igauge, isplit=1)
+    o = Oracle(prob)
+    w = C.smooth_wfn_for(prob, o.lcic)
+    o.set_wfn0(w)
+    o.h1itr_gen(DT / 2)
+    strength = np.array(C.LF_VEL if igauge else C.LF_LEN) * (1.0 if igauge else 10.0)
+
+    def context():
+        hp = td1c_amd.HProd(prob)
+        hp.set_wfn0(w)
+        hp.h1itr_gen(DT)
+        return hp
+
+    kept, terms = context(), set()
+    for k, scale in enumerate(SWITCHED):
+        ref, n = o.h1itr_prop(strength * scale, DT / 2, w)
+        terms.add(n)
+        d = kept.to_device(w)
+        kept.h1itr_prop(strength * scale, d)
+        fresh, e = context(), kept.to_device(w)
+        fresh.h1itr_prop(strength * scale, e)
+        torch.cuda.synchronize()
+        got = d.cpu().numpy()
+        assert np.array_equal(got, e.cpu().numpy()), (k, scale)
+        assert _rel(got, ref) < 1e-11, (k, scale, n)
+        fresh.close()
+    kept.close()
+    assert min(terms) <= 2 and max(terms) == 20 and len(terms) >= 4, terms
+
+
+def test_a_longer_series_costs_its_terms(gpu_lib):
+    """A series much longer than those before it costs what it costs when
+    the last one was as long, within a factor of 5 (some host waits more;
+    finished by one block on the device it took 95 times as long)."""
+    import time
+
+    import torch
+    import td1c_amd
+
+    prob = C.Problem(nfe=60, ndvr=20, rmax=120.0, lmax1=31, lmax2=62, znuc=10.0, ndcore=5, nel_alpha=5, nel_beta=5,
+                     lval=[0] * 5, igauge=1, isplit=1)
+    hp = td1c_amd.HProd(prob)
+    w = hp.to_device(C.smooth_wfn_for(prob, hp.lcic))
+    hp.h1itr_gen(DT)
+    weak, strong = np.array(C.LF_VEL) * 1e-3, np.array(C.LF_VEL) * 30.0
+
+    def seconds(lf):
+        d = w.clone()
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        hp.h1itr_prop(lf, d)
+        torch.cuda.synchronize()
+        return time.perf_counter() - t
+
+    seconds(strong)
+    after_weak, after_strong = [], []
+    for _ in range(3):
+        for _ in range(150):
+            seconds(weak)
+        after_weak.append(seconds(strong))
+        after_strong.append(min(seconds(strong) for _ in range(3)))
+    hp.close()
+    assert min(after_weak) < 5.0 * min(after_strong), (after_weak, after_strong)
