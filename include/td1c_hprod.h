@@ -432,13 +432,13 @@ int td1c_h1itr_gen(td1c_ctx* ctx, double dtime, int maxcyc, double thresh);
  * reference evaluates at t + dt/4 (first half step) or t + 3dt/4 (second).
  * The first check of the series (on x_0, norm ~1 per orbital) counts the
  * dynamical orbitals only.  Enqueued on `stream`; td1c_h1itr_gen first.
- * The call enqueues as many terms as the last series took and the
- * convergence test, waits for its result (a busy wait of up to 2 ms, then the
- * stream's own) and enqueues more until the series has converged.  The half
- * steps of td1c_propagate and the denominator series of the exponential
- * propagators do the same under stream launches (those calls return after the
- * last series, what follows it still on its way); under graph capture every
- * term is enqueued and nothing waits. */
+ * The call returns when the half step is done: it enqueues as many terms as
+ * the last series took and the convergence test, waits for its result (a
+ * busy wait of up to 2 ms, then the stream's own) and enqueues more until the
+ * series has converged.  The half steps of td1c_propagate and the denominator
+ * series of the exponential propagators wait in the same way under stream
+ * launches (those calls return after the last series, what follows it still
+ * on its way); under graph capture every term is enqueued and nothing waits. */
 int td1c_h1itr_prop(td1c_ctx* ctx, const double* lfield, double* d_wfn, void* stream);
 
 /* nstep steps (+ mask) from time t0 with the stage fields evaluated on the

@@ -2247,6 +2247,8 @@ int td1c_h1itr_prop(td1c_ctx* c, const double* lfield, double* d_wfn, void* stre
   int rc = enqueue_h1itr(c, c->lf_cn.p, reinterpret_cast<double2*>(d_wfn), s);
   if (rc) return rc;
   HIP_TRY(hipGetLastError());
+  // lfield is the caller's, and its next call may be on another stream
+  HIP_TRY(hipStreamSynchronize(s));
   return 0;
 }
 

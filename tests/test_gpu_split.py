@@ -269,3 +269,30 @@ def test_a_longer_series_costs_its_terms(gpu_lib):
         after_strong.append(min(seconds(strong) for _ in range(3)))
     hp.close()
     assert min(after_weak) < 5.0 * min(after_strong), (after_weak, after_strong)
+
+
+def test_half_step_is_done_on_return(gpu_lib):
+    """td1c_h1itr_prop returns with its stream idle, also when it expects the
+    length of the series: the field may be the caller's temporary, and the
+    next call may come on another stream (here: half steps on two streams in
+    turn, without events, give the bits of one stream)."""
+    import torch
+    import td1c_amd
+
+    prob = C.ne_small(isplit=1)
+    hp = td1c_amd.HProd(prob)
+    w = C.smooth_wfn_for(prob, hp.lcic)
+    hp.set_wfn0(w)
+    hp.h1itr_gen(DT)
+    ref, d = hp.to_device(w), hp.to_device(w)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(6):
+        hp.h1itr_prop(C.LF_VEL, ref)
+    torch.cuda.synchronize()
+    for k in range(6):
+        s = streams[k % 2]
+        hp.h1itr_prop(C.LF_VEL, d, stream=s.cuda_stream)
+        assert s.query(), k
+    assert np.array_equal(d.cpu().numpy(), ref.cpu().numpy())
+    hp.close()
