@@ -296,7 +296,7 @@ struct td1c_batch {
   int device = 0;
   bool use_graph = true;
   int ob_shape = 2, ob_lc = 2;  // element one-body launch shape of the batch
-  int tvar = 1;                 // register-blocked transform shape of the batch
+  int tvar = 1;                 // rows per block of the batch's transforms (0: 16, 1: 8)
   struct Site {
     LaunchRec proto;  // kind, variant and block of every member's launch
     int total = 0;    // blocks over all members
@@ -1256,7 +1256,7 @@ int td1c_ctx_create(const td1c_problem* prob, td1c_ctx** out) {
   if (rc) return rc;
   rc = autotune_onebody(c.get());
   if (rc) return rc;
-  if (const char* tv = std::getenv("TD1C_TVAR")) c->tvar = std::max(0, std::min(5, std::atoi(tv)));
+  if (const char* tv = std::getenv("TD1C_TVAR")) c->tvar = std::max(0, std::min(1, std::atoi(tv)));
   *out = c.release();
   return 0;
 }

@@ -142,6 +142,20 @@ def test_batch_autotuned_shapes_give_the_same_bits(gpu_lib):
         hp.close()
 
 
+@pytest.mark.parametrize("value,variant", [("-1", 0), ("0", 0), ("1", 1), ("5", 1)])
+def test_batch_transform_shape_from_the_environment(gpu_lib, monkeypatch, value, variant):
+    """TD1C_TVAR: one of the two shapes, in the batch's report and trials too."""
+    import td1c_amd
+
+    monkeypatch.setenv("TD1C_TVAR", value)
+    hps, ws = _members([_he(4, 3)])
+    b = td1c_amd.Batch(hps)
+    assert b.info()["transform_variant"] == variant
+    b.autotune([hp.to_device(w) for hp, w in zip(hps, ws)], DT, _fields(1))
+    assert {t[2] for t in b.info()["tune"]["ms_per_step"]} == {0, 1}
+    b.close()
+
+
 def test_batch_of_three_orbital_members(gpu_lib):
     """Three doubly occupied orbitals (m = 0, 1, -1) per member, two grids
     and nuclear charges: the pair densities, exchange and X matrix of each
