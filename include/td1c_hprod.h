@@ -485,7 +485,8 @@ int td1c_batch_set_graph(td1c_batch* batch, int on);
 
 /* Launch shapes of the batch: the element one-body kernel's elements per
  * block (3, 6, 12) and l values per block, and the matrix-core
- * transform's variant (0: 16 radial rows per block, 1: 8);
+ * transform's variant (0: 16 radial rows per block, 1: 8, which members with
+ * more than 200 l, L or theta values take either way);
  * every choice gives the same bits. */
 int td1c_batch_set_shapes(td1c_batch* batch, int elements_per_block, int l_per_block, int transform_variant);
 

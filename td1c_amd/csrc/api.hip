@@ -297,6 +297,7 @@ struct td1c_batch {
   bool use_graph = true;
   int ob_shape = 2, ob_lc = 2;  // element one-body launch shape of the batch
   int tvar = 1;                 // rows per block of the batch's transforms (0: 16, 1: 8)
+  bool tvar_free = true;        // both fit (td1c_batch_create)
   struct Site {
     LaunchRec proto;  // kind, variant and block of every member's launch
     int total = 0;    // blocks over all members
@@ -3267,7 +3268,11 @@ int td1c_batch_create(td1c_ctx* const* members, int n, td1c_batch** out) {
   td1c_batch* b = new td1c_batch();
   b->mem.assign(members, members + n);
   b->device = c0->device;
-  b->tvar = c0->tvar;
+  // the members' common transform shape: 16 rows of the longest contraction
+  // have to fit beside the job in 64 KB of LDS (57 KB at 200 values)
+  for (td1c_ctx* c : b->mem)
+    if (std::max({c->S.L1, c->S.L2, c->S.nlat}) > 200) b->tvar_free = false;
+  b->tvar = b->tvar_free ? c0->tvar : 1;
   *out = b;
   return 0;
 }
@@ -3293,7 +3298,7 @@ int td1c_batch_set_shapes(td1c_batch* b, int elements_per_block, int l_per_block
   if (transform_variant != 0 && transform_variant != 1) return fail(-1, "transform_variant must be 0 or 1");
   b->ob_shape = shape;
   b->ob_lc = l_per_block;
-  b->tvar = transform_variant;
+  b->tvar = b->tvar_free ? transform_variant : 1;
   b->key.clear();  // record again
   return 0;
 }
@@ -3502,8 +3507,6 @@ int batch_record(td1c_batch* b, const std::vector<Pulse>& pulses, int rk_order, 
                  int apply_mask) {
   const int nmem = (int)b->mem.size();
   std::vector<std::vector<LaunchRec>> recs(nmem);
-  int kmax = 0;  // the longest contraction decides the members' common transform shape (LDS)
-  for (td1c_ctx* c : b->mem) kmax = std::max({kmax, c->S.L2, c->S.nlat});
   for (int m = 0; m < nmem; ++m) {
     td1c_ctx* c = b->mem[m];
     int ns;
@@ -3515,7 +3518,7 @@ int batch_record(td1c_batch* b, const std::vector<Pulse>& pulses, int rk_order, 
     c->tpath = 2;  // the matrix-core transforms (their batched form)
     c->ob_shape = b->ob_shape;
     c->ob_lc = b->ob_lc;
-    c->tvar = kmax > 200 ? 1 : b->tvar;
+    c->tvar = b->tvar;
     c->capturing = true;  // no per-kernel timing events
     active_recorder() = &R;
     launch_field_stages(pulses[m], c->clock.p, sn, c->lf_dev.p, c->side[1]);
@@ -3880,7 +3883,7 @@ int td1c_batch_autotune(td1c_batch* b, const td1c_field* fields, int rk_order, d
       rc = trial(shape, lc, t0);
       if (rc) break;
     }
-  if (!rc) rc = trial(bs, bl, 1 - t0);
+  if (!rc && b->tvar_free) rc = trial(bs, bl, 1 - t0);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   b->ob_shape = bs;

@@ -142,6 +142,36 @@ def test_batch_autotuned_shapes_give_the_same_bits(gpu_lib):
         hp.close()
 
 
+@pytest.mark.parametrize("lmax1,lmax2,free", [(200, 40, False), (230, 20, False), (40, 200, False), (20, 199, True)])
+def test_batch_transform_shape_of_long_contractions(gpu_lib, lmax1, lmax2, free):
+    """More than 200 l, L or theta values: 16 rows of such a contraction
+    leave no room in 64 KB of LDS (l -> theta contracts over l, lmax1 + 1 of
+    them), so the batch runs, tries and reports 8 rows whatever is asked for;
+    up to 200 the choice stands.  The same bits either way."""
+    import torch
+    import td1c_amd
+
+    prob = Problem(nfe=3, ndvr=20, rmax=6.0, lmax1=lmax1, lmax2=lmax2, znuc=2.0, ndcore=1, nel_alpha=1, nel_beta=1,
+                   igauge=1, isplit=1)
+    hps = [td1c_amd.HProd(p) for p in (prob, _he(4, 3))]
+    ws = [C.wfn_for(hp.prob, hp.lcic) for hp in hps]  # (the bound shapes r^(l+1) underflow at these l)
+    b = td1c_amd.Batch(hps)
+    states = []
+    for variant in (0, 1):
+        b.set_shapes(6, 2, variant)
+        assert b.info()["transform_variant"] == (variant if free else 1)
+        d = [hp.to_device(w) for hp, w in zip(hps, ws)]
+        b.propagate(d, 20.0, DT, 1, _fields(2))
+        torch.cuda.synchronize()
+        states.append([x.cpu().numpy() for x in d])
+    for x, y in zip(*states):
+        assert np.isfinite(x).all() and np.array_equal(x, y)
+    b.autotune([hp.to_device(w) for hp, w in zip(hps, ws)], DT, _fields(2))
+    tried = [t[2] for t in b.info()["tune"]["ms_per_step"]]
+    assert len(tried) == (13 if free else 12) and set(tried) == ({0, 1} if free else {1}), tried
+    b.close()
+
+
 @pytest.mark.parametrize("value,variant", [("-1", 0), ("0", 0), ("1", 1), ("5", 1)])
 def test_batch_transform_shape_from_the_environment(gpu_lib, monkeypatch, value, variant):
     """TD1C_TVAR: one of the two shapes, in the batch's report and trials too."""
