@@ -88,9 +88,13 @@ __device__ __forceinline__ double2 gather_E(const IslandArgs& a, const CiView& v
 // whole block (n <= 8).  A round rotates the disjoint pairs of a round-robin
 // schedule together: lane (slot, k) of the first 32 owns row or column k of
 // pair slot, lanes 32..63 the rows of U.  A serial chain: one lane sweeping
-// the pairs one by one took about 200 us for n = 6.  Ends when the squared
-// off-diagonal is below 1e-34 of the squared diagonal (rounding).
-__device__ void herm_eig(int n, double2* A, double* w, double2* U, double* s_off) {
+// the pairs one by one took about 200 us for n = 6.  Ends when each squared
+// element is below 1e-34 of the product of its two diagonal ones (rounding):
+// weakly occupied orbitals make a graded matrix, whose small eigenvalues the
+// rotations give to full relative accuracy if they run until then.  (Measured
+// against the squared diagonal of all, the inverse lost up to 3e-10 of its norm
+// at occupations down to 1e-12, where this loses 4e-15.)
+__device__ void herm_eig(int n, double2* A, double* w, double2* U, int* s_more) {
   const int tid = threadIdx.x;
   for (int i = tid; i < n * n; i += kT) U[i] = make_double2(i % n == i / n ? 1.0 : 0.0, 0.0);
   const int N = n + (n & 1);  // players of the schedule; index n of an odd n sits out
@@ -99,21 +103,16 @@ __device__ void herm_eig(int n, double2* A, double* w, double2* U, double* s_off
     __syncthreads();
     if (tid < 64) {
       const int i = tid & 7, j = tid >> 3;
-      double off = 0.0, dia = 0.0;
-      if (i < n && j < n) {
+      bool more = false;
+      if (i < n && j < n && i != j) {
         const double2 z = A[i + n * j];
-        const double m = z.x * z.x + z.y * z.y;
-        if (i == j) dia = m;
-        else off = m;
+        more = !(z.x * z.x + z.y * z.y <= fmax(1e-34 * fabs(A[i + n * i].x * A[j + n * j].x), 1e-300));
       }
-      for (int o = 32; o > 0; o >>= 1) {
-        off += __shfl_xor(off, o, 64);
-        dia += __shfl_xor(dia, o, 64);
-      }
-      if (tid == 0) *s_off = off <= 1e-34 * dia ? 0.0 : 1.0;
+      const unsigned long long any = __ballot(more);
+      if (tid == 0) *s_more = any != 0;
     }
     __syncthreads();
-    if (*s_off == 0.0) break;
+    if (*s_more == 0) break;
     for (int round = 0; round < N - 1; ++round) {
       // the pair of this slot: the fixed player N-1 meets `round`, the others
       // pair off symmetrically around it
@@ -204,10 +203,11 @@ __device__ __forceinline__ void put_den1(const IslandArgs& a, int e, double2 s, 
 // rden = D^-1 and rrden = (2 - D)^-1, regularised, from den1 in LDS
 __device__ void put_inverses(const IslandArgs& a, const double2* s_d1) {
   __shared__ double2 s_A[kN2], s_U[kN2];
-  __shared__ double s_w[kMaxAct], s_off;
+  __shared__ double s_w[kMaxAct];
+  __shared__ int s_more;
   const int n = a.nact;
   for (int e = threadIdx.x; e < n * n; e += kT) s_A[e] = s_d1[e];
-  herm_eig(n, s_A, s_w, s_U, &s_off);
+  herm_eig(n, s_A, s_w, s_U, &s_more);
   for (int e = threadIdx.x; e < n * n; e += kT) {
     const double2 r = inv_entry(n, a.throcc1, s_U, s_w, e);
     a.rden[e] = r;
@@ -224,7 +224,7 @@ __device__ void put_inverses(const IslandArgs& a, const double2* s_d1) {
     const double d = e % n == e / n ? 2.0 : 0.0;
     s_A[e] = make_double2(d - s_d1[e].x, -s_d1[e].y);
   }
-  herm_eig(n, s_A, s_w, s_U, &s_off);
+  herm_eig(n, s_A, s_w, s_U, &s_more);
   for (int e = threadIdx.x; e < n * n; e += kT) a.rrden[e] = inv_entry(n, a.throcc2, s_U, s_w, e);
 }
 

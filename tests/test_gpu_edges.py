@@ -57,6 +57,29 @@ def test_partitions(gpu_lib, nfc, ndc, nact, nel, precision):
     assert hprod_error(prob, C.LF_VEL) < (1e-5 if precision else 1e-11)
 
 
+# occupations graded over ten decades (the CI coefficients of orbital i scaled by
+# 10^(-5 i / (n - 1))), for the regularised inverse of the 1-RDM: the weakly
+# occupied orbitals dominate the derivative, and a Jacobi sweep that stops at a
+# fraction of the largest occupation leaves 5e-11 in it (seed 87)
+@pytest.mark.parametrize("n,seed", [(8, 87), (8, 91), (6, 31), (4, 125)])
+def test_graded_occupations(gpu_lib, n, seed):
+    import torch
+
+    prob = Problem(nfe=3, ndvr=20, rmax=9.0, lmax1=3, lmax2=6, znuc=2.0, nact=n, nel_alpha=1, nel_beta=1, lval=[0] * n,
+                   igauge=1)
+    o = Oracle(prob)
+    w = C.wfn_for(prob, o.lcic)
+    rng = np.random.default_rng(seed)
+    scale = 10.0 ** np.linspace(0, -5, n)
+    ci = scale[:, None] * (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))) * scale
+    w[-o.lcic:] = ci.ravel() / np.linalg.norm(ci)
+    ref = o.htot(1.0, C.LF_VEL, w)
+    hp = td1c_amd.HProd(prob)
+    got = hp.htot(1.0, C.LF_VEL, hp.to_device(w))
+    torch.cuda.synchronize()
+    assert np.linalg.norm(got.cpu().numpy() - ref) < 1e-11 * np.linalg.norm(ref)
+
+
 # the element one-body kernel at orders other than 20 (rows padded to 16, 24
 # and 32) and element counts that end inside a block, both gauges, a frozen
 # core beside m = 0 and 1; the half step's right-hand sides with it
