@@ -2820,7 +2820,7 @@ int enqueue_etd_step(td1c_ctx* c, const double* d_lf, double2* wfn, int apply_ma
     }
   };
   // the denominator factors of R on the dynamical rows of orb, in place
-  int series_err = 0;  // a failed allocation of enqueue_series
+  int series_err = 0;  // a failure of enqueue_series
   auto denom = [&](const td1c_ctx::EtdRat& R) {
     for (int i = 0; i < R.dimd; ++i) {
       if (R.tab[i] < 0) continue;

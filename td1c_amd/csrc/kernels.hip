@@ -1194,10 +1194,11 @@ void launch_transform_t(int mode, const TI* in, TO* out, const LegendreMats& M, 
     record_launch(kRecLegendre, var, dim3(r.ntile), 256, (size_t)8 * J.KS * 16 * rnt * (F32 ? 4 : 8), r);
     return;
   }
-  // the matrix cores from 16 columns on; below, the vector form (whole hprods
-  // of 1-9 orbitals on 240-2400 points: lmax1 7 in length gauge 102 us by the
-  // vector form against 117, lmax1 31 378 against 414 (9 orbitals), lmax1 63
-  // 757 against 974; the rest within 5 %)
+  // the matrix cores from 16 columns on; below, the vector form.  us per FP64
+  // hprod of 9 orbitals on 2399 points, vector form / matrix cores: lmax1 5
+  // 114 / 136, 7 129 / 149, 11 163 / 173, 15 196 / 199, 31 407 / 372, 63
+  // 977 / 755 (lmax2 = 2 lmax1; complex64 alike: 7 120 / 131, 15 166 / 167, 63
+  // 738 / 529); one orbital is bound by its launches either way
   const bool mfma = C >= 16;
   if (path == 1 || (path == 0 && !mfma)) {
     const int rt = (nr + 63) / 64;
@@ -1619,6 +1620,12 @@ void launch_mfprod(const T* orbg, const T* vg, T* gorbg, T* v2orbg, const MfArgs
     else hipLaunchKernelGGL((k_mfprod_quad<0, T>), gq, dim3(bt), 0, s, orbg, vg, gorbg, v2orbg, a);
     return;
   }
+  // The partitions held in registers: every number of doubly occupied orbitals
+  // up to 16, and active orbitals beside at most one frozen and one dynamical
+  // core as far as nfun <= 9 and (both cores) nact <= 4.  Each costs seconds of
+  // build and tens of KB of library in its two precisions.  The others keep the
+  // generic kernel: frozen cores beside doubly occupied orbitals alone, two
+  // frozen cores, two dynamical cores beside active orbitals.
   switch (key) {
     // dynamical cores only
     MF_CASE(0, 1, 0) MF_CASE(0, 2, 0) MF_CASE(0, 3, 0) MF_CASE(0, 4, 0) MF_CASE(0, 5, 0) MF_CASE(0, 6, 0)

@@ -40,7 +40,7 @@ def cas_fc_small(**kw):
 
 
 def he_n16(**kw):
-    # ndvr = 16 runs the band one-body kernel instead of the element kernel
+    # ndvr = 16: the element one-body kernel with its rows at their bound of 16
     return Problem(nfe=10, ndvr=16, rmax=30.0, lmax1=5, lmax2=10, znuc=2.0, ndcore=1,
                    nel_alpha=1, nel_beta=1, **kw)
 
@@ -53,7 +53,7 @@ def he_long(**kw):
 
 
 def dc4_small(**kw):
-    # four doubly occupied orbitals: the generic theta-grid mean-field kernel
+    # four doubly occupied orbitals in the mean-field kernel
     return Problem(nfe=6, ndvr=20, rmax=18.0, lmax1=5, lmax2=10, znuc=8.0, ndcore=4,
                    nel_alpha=4, nel_beta=4, **kw)
 

@@ -1,8 +1,8 @@
 """cletdrb (exponential Rosenbrock RK4 with Pade phi functions, the
 reference's default prop_type) on the GPU against the oracle's
 orc_etdrb_step: He, three-orbital, frozen-core + CAS and CAS problems in both
-gauges, the element (ndvr = 20) and band (ndvr = 16, 10) one-body paths, real
-and imaginary time, FP64 and the complex64 mean field.  Two steps at dt =
+gauges, ndvr = 20 and the padded rows of other orders (16, 10), real and
+imaginary time, FP64 and the complex64 mean field.  Two steps at dt =
 0.01 from a bound-state-like state in a sin^2 pulse: FP64 relative L2 1e-10,
 mixed 1e-6."""
 import numpy as np
@@ -68,8 +68,8 @@ def test_etdrb_steps_match_oracle(gpu_lib, name, igauge, precision):
 
 
 def test_etdrb_imaginary_time_matches_oracle(gpu_lib):
-    """icomp = 0 (no Neumann series in the denominators; tunit = -1), band
-    one-body path (ndvr = 10)."""
+    """icomp = 0 (no Neumann series in the denominators; tunit = -1), one-body
+    rows padded from ndvr = 10."""
     import torch
     import td1c_amd
 

@@ -18,7 +18,7 @@ def _rel(a, b):
 
 
 CASES = [("he_small", C.LF_LEN), ("dc3_small", C.LF_LEN), ("ne_small", C.LF_VEL), ("cas_fc_small", C.LF_VEL),
-         ("cas_small", C.LF_LEN), ("he_n16", C.LF_VEL)]  # ndvr = 16: the band right-hand-side kernel
+         ("cas_small", C.LF_LEN), ("he_n16", C.LF_VEL)]  # ndvr = 16: rows of another length
 
 
 @pytest.mark.parametrize("name,lf", CASES)
@@ -45,7 +45,7 @@ def test_split_hprod_matches_oracle(gpu_lib, name, lf):
 def test_h1itr_half_step_matches_oracle(gpu_lib, name, lf):
     """td1c_h1itr_prop (element Schur solve + series with a device
     convergence test) against h1itr_prop (band LU), twice in a row on the
-    same context (the flag and the ticket are reused)."""
+    same context (the flag is reused)."""
     import torch
     import td1c_amd
     from oracle.oracle import Oracle
