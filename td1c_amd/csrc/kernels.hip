@@ -1622,7 +1622,7 @@ void launch_mfprod(const T* orbg, const T* vg, T* gorbg, T* v2orbg, const MfArgs
   }
   // The partitions held in registers: every number of doubly occupied orbitals
   // up to 16, and active orbitals beside at most one frozen and one dynamical
-  // core as far as nfun <= 9 and (both cores) nact <= 4.  Each costs seconds of
+  // core as far as nfun <= 9 and (beside both) nact <= 4.  Each costs seconds of
   // build and tens of KB of library in its two precisions.  The others keep the
   // generic kernel: frozen cores beside doubly occupied orbitals alone, two
   // frozen cores, two dynamical cores beside active orbitals.
